@@ -192,3 +192,34 @@ def test_bf16_rounding_instruction_against_the_oracle(dev, first):
     x = np.arange(first, first + count, dtype=np.uint64).astype(np.uint32).view(np.float32)
     assert np.array_equal(bits_of(bits), O.bf16_round(x))
     assert bad.cpu().numpy().view(np.uint32).tolist() == [0, 0xFFFFFFFF]
+
+
+@pytest.mark.parametrize("fmt", ["fp4_e2m1", "fp6_e2m3", "fp6_e3m2"])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16, torch.float32])
+def test_quantize_vector_kernel_matches_scalar_kernel(dev, fmt, xdt):
+    """Aligned whole blocks (vector kernel) against the same values one element off (scalar kernel): every
+    16-bit pattern, in blocks of one magnitude range and in mixed blocks, with infinities, NaN, zeros,
+    subnormals and exact ties."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    if xdt is torch.float32:
+        bits = torch.randint(-2**31, 2**31 - 1, (65536,), device=dev, generator=g).to(torch.int32)
+        bits[::7] &= ~0xFFFFF  # few significant bits: ties between codes
+        every = bits.view(torch.float32)
+    else:
+        every = torch.arange(-32768, 32768, device=dev, dtype=torch.int32).to(torch.int16).view(xdt)
+    order = every.float().abs().nan_to_num(nan=3e38).argsort()
+    mixed = torch.randperm(65536, device=dev, generator=g)
+    ties = (torch.randint(-32, 33, (8192,), device=dev, generator=g) / 8.0
+            * torch.exp2(torch.randint(-12, 12, (8192,), device=dev, generator=g).float() // 1)).to(xdt)
+    zeros = torch.zeros(64, dtype=xdt, device=dev)
+    zeros[33] = -0.0
+    x = torch.cat([every[order], every[mixed], ties, zeros])
+    x = x.reshape(-1, 64)
+    store = torch.empty(x.numel() + 1, dtype=xdt, device=dev)
+    shifted = store[1:].view(x.shape)
+    shifted.copy_(x)
+    assert x.data_ptr() % 16 == 0 and shifted.data_ptr() % 16 != 0
+    fast, slow = quantize_mx(x, fmt), quantize_mx(shifted, fmt)
+    assert torch.equal(fast.scales.view(torch.uint8), slow.scales.view(torch.uint8))
+    assert torch.equal(fast.data, slow.data)
