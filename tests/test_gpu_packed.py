@@ -223,3 +223,27 @@ def test_quantize_vector_kernel_matches_scalar_kernel(dev, fmt, xdt):
     fast, slow = quantize_mx(x, fmt), quantize_mx(shifted, fmt)
     assert torch.equal(fast.scales.view(torch.uint8), slow.scales.view(torch.uint8))
     assert torch.equal(fast.data, slow.data)
+
+
+@pytest.mark.parametrize("fmt", list(FORMATS))
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape,bs", [((64, 1024), 32), ((33, 516), 32), ((257, 40), 24), ((5, 7), 3), ((2049,), 32),
+                                      ((3, 4096), 128)])
+def test_unpack_vector_kernel_matches_scalar_kernel(dev, fmt, out, shape, bs):
+    """Aligned storage (vector kernel) against the same bytes at an odd address (scalar kernel), bit for bit:
+    rows and scale blocks that end inside a chunk, tails, E8M0 extremes, infinite and NaN scales."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(4)
+    count, sshape = math.prod(shape), shape[:-1] + (-(-shape[-1] // bs),)
+    nbytes = (count * FORMATS[fmt][0] + 7) // 8
+    store = torch.randint(0, 256, (nbytes + 1,), dtype=torch.uint8, device=dev, generator=g)
+    data, odd = store[1:].clone(), store[1:]
+    e8 = torch.randint(0, 256, sshape, dtype=torch.uint8, device=dev, generator=g).view(torch.float8_e8m0fnu)
+    f32 = torch.randn(sshape, device=dev, generator=g) * 10
+    f32.view(-1)[0] = float("inf")
+    f32.view(-1)[-1] = float("nan")
+    f32.view(-1)[f32.numel() // 2] = -1e36
+    for scales in (None, e8, f32, f32.to(torch.float16), f32.to(torch.bfloat16)):
+        fast = PackedTensor(data, fmt, shape, scales, bs).unpack(out)
+        slow = PackedTensor(odd, fmt, shape, scales, bs).unpack(out)
+        assert np.array_equal(bits_of(fast), bits_of(slow))
