@@ -643,6 +643,46 @@ def test_gemm_w_int4_one_hot_is_exact(dev, fmt, bs):
     assert np.array_equal(c, deq[:, cols].T.astype(np.float32))
 
 
+# one shape per tile of the one-tile kernels (ragged in M and N), step counts that the K groups of a
+# workgroup do not divide, and a single step
+@pytest.mark.parametrize("fmt,sdt,bs", [("fp4_e2m1", "e8m0", 32), ("fp6_e2m3", "e8m0", 32), ("fp6_e3m2", "none", 32),
+                                        ("int4", torch.float16, 128), ("uint4", torch.bfloat16, 64),
+                                        ("int4", torch.float32, 32), ("uint4", torch.float32, 128), ("int4", None, 32)])
+@pytest.mark.parametrize("mnk", [(17, 33, 128), (40, 1000, 640), (70, 4100, 384), (130, 4100, 1152), (200, 6150, 640),
+                                 (500, 6150, 384), (1030, 6150, 256)])
+def test_gemm_w_one_tile_shapes(dev, fmt, sdt, bs, mnk):
+    m, n, k = mnk
+    rng = np.random.default_rng(m + n + k + bs)
+    if isinstance(sdt, str):
+        w, deq = make_weight(dev, fmt, n, k, sdt, rng)
+        a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(dev).to(torch.bfloat16)
+    else:
+        w, deq = int4_weight(dev, fmt, n, k, sdt, bs, rng)
+        a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float16)).to(dev)
+    c = matmul_nt(a, w, scope="ThreadGroup", dtype=torch.float32)
+    ref = a.double() @ torch.from_numpy(np.asarray(deq, np.float64)).to(dev).T
+    # fp32 sums of k exact products: at most k roundings of 2^-24 of the partial sums, in practice sqrt(k)
+    bound = 4 * k ** 0.5 * 2.0 ** -24 * (a.double().abs() @ torch.from_numpy(np.abs(np.asarray(deq, np.float64))).to(dev).T)
+    assert bool(((c.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("fmt", ["fp4_e2m1", "fp6_e2m3", "int4"])
+def test_gemm_w_nan_scales_stay_in_their_row(dev, fmt):
+    """K groups past the last step read nothing: a NaN in the next row's first scale stays out."""
+    m, n, k = 20, 96, 640  # 5 steps, 4 K groups per workgroup
+    rng = np.random.default_rng(8)
+    if fmt == "int4":
+        w, _ = int4_weight(dev, fmt, n, k, torch.float16, 128, rng)
+        w.scales[1::2, 0] = float("nan")
+        a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float16)).to(dev)
+    else:
+        w, _ = make_weight(dev, fmt, n, k, "e8m0", rng)
+        w.scales.view(torch.uint8)[1::2, 0] = 255
+        a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(dev).to(torch.bfloat16)
+    c = matmul_nt(a, w, scope="ThreadGroup", dtype=torch.float32)
+    assert bool(c[:, 0::2].isfinite().all()) and bool(c[:, 1::2].isnan().all())
+
+
 def test_gemm_w_int4_prefill_shape(dev):
     """Attention-projection prefill shape: 512 tokens x fp16 [512, 4096] times INT4 g128
     fp16-scale weights [6144, 4096] (q, k and v rows stacked), fp16 out."""
