@@ -650,9 +650,8 @@ template <int FMT, bool SCALED, bool SWIGLU = false>
 int launch_gemm_w(const void* a, int64_t lda, const void* w, const void* scales, int64_t m, int64_t n, int64_t k,
                   void* c, int cdt, int64_t ldc, hipStream_t stream, int splits = 1, float* part = nullptr) {
   const int64_t tiles = ((m + kWM - 1) / kWM) * ((n + kWN - 1) / kWN);
-  const int cus = stream_cu_count(stream);
-  if (!SWIGLU && splits == 1 && !part && k % kVKMultiple == 0 && cus >= 8 && tiles >= cus) {
-    // at least one round of tiles: persistent, one workgroup per CU (a multiple of 8 of them)
+  if (!SWIGLU && !part) {  // persistent, one workgroup per CU (a multiple of 8 of them)
+    const int cus = stream_cu_count(stream);
     hipLaunchKernelGGL((gemm_w_stream<FMT, SCALED>), dim3((unsigned)(cus / 8 * 8)), dim3(512), 0, stream,
                        (const uint8_t*)a, (unsigned)(lda * 2), (const uint8_t*)w, (const uint8_t*)scales, (int)m,
                        (int)n, (int)k, c, cdt, ldc);
@@ -668,6 +667,30 @@ int launch_gemm_w(const void* a, int64_t lda, const void* w, const void* scales,
 }  // namespace tgm
 
 using namespace tgm;
+
+// At least one round of 128 x 256 tiles, and whole scale batches: the persistent kernel's products (and
+// gemm_w_mx's, for the SwiGLU form).  Smaller ones go to the one-tile kernels (figures in tgm_gemm_w_tile.h;
+// at one round exactly, FP4 2048 x 4096 x 4096: 56.2 us persistent, 57.5 us on one-tile 128 x 256).
+static bool whole_round(int64_t m, int64_t n, int64_t k, int cus) {
+  return k % kVKMultiple == 0 && cus >= 8 && ((m + kWM - 1) / kWM) * ((n + kWN - 1) / kWN) >= cus;
+}
+
+static WTileArgs tile_args(const void* a, int64_t lda, const void* w, const void* scales, int scale_dtype, int64_t m,
+                           int64_t n, int64_t k, void* c, int c_dtype, int64_t ldc) {
+  WTileArgs t{};
+  t.a = (const uint8_t*)a;
+  t.w = (const uint8_t*)w;
+  t.scales = (const uint8_t*)scales;
+  t.c = c;
+  t.ldc = ldc;
+  t.lda_bytes = (unsigned)(lda * 2);
+  t.M = (int)m;
+  t.N = (int)n;
+  t.K = (int)k;
+  t.cdt = c_dtype;
+  t.sdt = scale_dtype;
+  return t;
+}
 
 // tgm_gemm_w with K split over `splits` rows of workgroups (fp32 partials in `part`, summed by
 // gemm_split_reduce); splits == 1 with part == nullptr is the plain product.
@@ -696,25 +719,14 @@ static int gemm_w_impl(const void* a, int a_dtype, int64_t m, int64_t lda, const
     TGM_UNSUPPORTED("tgm_gemm_w: operands must be 16-byte and scales 4-byte aligned");
   const hipStream_t st = (hipStream_t)stream;
   const int64_t lda_eff = m > 1 ? lda : k;
-  WTileArgs t{};
-  t.a = (const uint8_t*)a;
-  t.w = (const uint8_t*)w;
-  t.scales = (const uint8_t*)scales;
-  t.c = c;
-  t.ldc = ldc;
-  t.lda_bytes = (unsigned)(lda_eff * 2);
-  t.M = (int)m;
-  t.N = (int)n;
-  t.K = (int)k;
-  t.cdt = c_dtype;
-  t.sdt = scale_dtype;
-  t.is_signed = fmt == TGM_FMT_INT4;
-  t.part = part;
-  t.steps_per_split = (int)((k / kWK + splits - 1) / splits);
   const int cus = stream_cu_count(st);
-  if (int4) return launch_gemm_w_tile_i4(t, block_size, splits, cus, st);
-  const int64_t tiles = ((m + kWM - 1) / kWM) * ((n + kWN - 1) / kWN);
-  if (!part && !(k % kVKMultiple == 0 && cus >= 8 && tiles >= cus)) return launch_gemm_w_tile_mx(t, fmt, cus, st);
+  if (int4 || (!part && !whole_round(m, n, k, cus))) {
+    WTileArgs t = tile_args(a, lda_eff, w, scales, scale_dtype, m, n, k, c, c_dtype, ldc);
+    t.is_signed = fmt == TGM_FMT_INT4;
+    t.part = part;
+    t.steps_per_split = (int)((k / kWK + splits - 1) / splits);
+    return int4 ? launch_gemm_w_tile_i4(t, block_size, splits, cus, st) : launch_gemm_w_tile_mx(t, fmt, cus, st);
+  }
   switch (fmt * 2 + (scaled ? 1 : 0)) {
     case TGM_FMT_FP4_E2M1 * 2 + 1: return launch_gemm_w<TGM_FMT_FP4_E2M1, true>(a, lda_eff, w, scales, m, n, k, c, c_dtype, ldc, st, splits, part);
     case TGM_FMT_FP4_E2M1 * 2: return launch_gemm_w<TGM_FMT_FP4_E2M1, false>(a, lda_eff, w, scales, m, n, k, c, c_dtype, ldc, st, splits, part);
@@ -879,6 +891,12 @@ extern "C" int tgm_gemm_w_swiglu(const void* a, int a_dtype, int64_t m, int64_t 
   if ((uintptr_t)a % 16 || (uintptr_t)w % 16 || (scaled && (uintptr_t)scales % 4))
     TGM_UNSUPPORTED("tgm_gemm_w_swiglu: operands must be 16-byte and scales 4-byte aligned");
   const int64_t lda_eff = m > 1 ? lda : k;
+  const int cus = stream_cu_count((hipStream_t)stream);
+  if (!whole_round(m, n, k, cus)) {  // the same kernels as tgm_gemm_w, so the same sums
+    WTileArgs t = tile_args(a, lda_eff, w, scales, scale_dtype, m, n, k, c, c_dtype, ldc);
+    t.swiglu = 1;
+    return launch_gemm_w_tile_mx(t, fmt, cus, (hipStream_t)stream);
+  }
   return scaled ? launch_gemm_w<TGM_FMT_FP4_E2M1, true, true>(a, lda_eff, w, scales, m, n, k, c, c_dtype, ldc,
                                                               (hipStream_t)stream)
                 : launch_gemm_w<TGM_FMT_FP4_E2M1, false, true>(a, lda_eff, w, scales, m, n, k, c, c_dtype, ldc,

@@ -72,6 +72,7 @@ struct WTileArgs {
   int M, N, K, cdt, sdt, is_signed;
   int steps_per_split;  // > 0: blockIdx.y takes that many K steps and writes its fp32 product to part [splits][M][N]
   float* part;
+  int swiglu;  // rows of W interleave gate and up: C has N / 2 columns, silu(gate) * up
 };
 
 // 16-bit values to LDS, one zero-extended dword per lane.
@@ -417,6 +418,8 @@ gemm_w_tile(WTileArgs p) {
     if (WK == 1 && p.part)
       store_tile32(acc[t], ep, lane, m0 + 32 * t, n0 + 32 * wn, p.M, p.N, p.part + (int64_t)blockIdx.y * p.M * p.N, TGM_F32,
                    p.N);
+    else if (!I4 && p.swiglu)
+      store_tile32_swiglu(acc[t], ep, lane, m0 + 32 * t, n0 + 32 * wn, p.M, p.N, p.c, p.cdt, p.ldc);
     else store_tile32(acc[t], ep, lane, m0 + 32 * t, n0 + 32 * wn, p.M, p.N, p.c, p.cdt, p.ldc);
   }
 }
@@ -436,8 +439,9 @@ int launch_w_tile(const WTileArgs& p, int splits, hipStream_t stream) {
 // decide, hold for K = 1024 to 14336), and lo2 .. hi2 for two (less than twice where two workgroups fit a
 // compute unit's LDS).  The smallest estimate wins, so a product takes the smallest tile that still gives
 // every compute unit one workgroup, and larger tiles, which read less per MFMA, as it grows.
+// Shapes that split K over wk waves want two K steps for each; shorter products go to the others.
 struct TileCost {
-  int bm, bn;
+  int bm, bn, wk;
   float lo, hi, lo2, hi2;
 };
 inline float tile_estimate(const TileCost& t, int64_t m, int64_t n, int64_t cus) {
@@ -448,12 +452,13 @@ inline float tile_estimate(const TileCost& t, int64_t m, int64_t n, int64_t cus)
   return (float)pairs * t.hi2 + tail;
 }
 template <int COUNT>
-int cheapest_tile(const TileCost (&table)[COUNT], int64_t m, int64_t n, int cus) {
-  int best = 0;
+int cheapest_tile(const TileCost (&table)[COUNT], int64_t m, int64_t n, int64_t k, int cus) {
+  int best = -1;
   float least = 0.f;
   for (int i = 0; i < COUNT; ++i) {
+    if (table[i].wk > 1 && k / kWtK < 2 * table[i].wk) continue;
     const float e = tile_estimate(table[i], m, n, cus > 0 ? cus : 256);
-    if (i == 0 || e < least) {
+    if (best < 0 || e < least) {
       best = i;
       least = e;
     }

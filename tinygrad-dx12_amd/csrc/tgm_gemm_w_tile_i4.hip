@@ -6,17 +6,17 @@ namespace tgm {
 // us at K = 4096 with fp16 scales per 128 and per 32 (every 32 K-elements the partial sums cost FA x 16 FMAs
 // per wave, so the small tiles pay more for them).
 static constexpr TileCost kI4Tiles[] = {
-    {32, 32, 9.0f, 10.3f, 17.5f, 18.1f},   {32, 64, 9.8f, 11.3f, 19.9f, 22.3f},   {64, 64, 15.9f, 18.6f, 32.0f, 33.6f},
-    {64, 128, 21.3f, 25.1f, 43.0f, 48.0f}, {64, 128, 23.6f, 28.5f, 36.0f, 43.4f}, {128, 256, 48.0f, 67.6f, 111.0f, 120.0f}};
+    {32, 32, 4, 9.0f, 10.3f, 17.5f, 18.1f},   {32, 64, 4, 9.8f, 11.3f, 19.9f, 22.3f},   {64, 64, 2, 15.9f, 18.6f, 32.0f, 33.6f},
+    {64, 128, 2, 21.3f, 25.1f, 43.0f, 48.0f}, {64, 128, 1, 23.6f, 28.5f, 36.0f, 43.4f}, {128, 256, 1, 48.0f, 67.6f, 111.0f, 120.0f}};
 static constexpr TileCost kI4Tiles32[] = {
-    {32, 32, 12.2f, 13.8f, 24.4f, 25.5f},  {64, 32, 16.7f, 19.9f, 34.7f, 35.8f},  {64, 64, 23.9f, 26.3f, 48.5f, 49.0f},
-    {64, 128, 28.6f, 36.2f, 67.0f, 70.0f}, {128, 256, 73.0f, 88.0f, 153.0f, 160.0f}};
+    {32, 32, 4, 12.2f, 13.8f, 24.4f, 25.5f},  {64, 32, 4, 16.7f, 19.9f, 34.7f, 35.8f},  {64, 64, 2, 23.9f, 26.3f, 48.5f, 49.0f},
+    {64, 128, 2, 28.6f, 36.2f, 67.0f, 70.0f}, {128, 256, 1, 73.0f, 88.0f, 153.0f, 160.0f}};
 
 template <int KIND>
 static int launch_kind(const WTileArgs& p, int splits, int cus, hipStream_t st) {
   // split K keeps the largest tile: its callers split products whose 128 x 256 tiles are few
   if constexpr (kind_group(KIND) == 32) {
-    switch (p.part ? 4 : cheapest_tile(kI4Tiles32, p.M, p.N, cus)) {
+    switch (p.part ? 4 : cheapest_tile(kI4Tiles32, p.M, p.N, p.K, cus)) {
       case 0: return launch_w_tile<KIND, 1, 1, 4, 3>(p, 1, st);
       case 1: return launch_w_tile<KIND, 2, 1, 4, 2>(p, 1, st);
       case 2: return launch_w_tile<KIND, 2, 2, 2, 3>(p, 1, st);
@@ -24,7 +24,7 @@ static int launch_kind(const WTileArgs& p, int splits, int cus, hipStream_t st) 
       default: return launch_w_tile<KIND, 4, 8, 1, 2>(p, splits, st);
     }
   } else {
-    switch (p.part ? 5 : cheapest_tile(kI4Tiles, p.M, p.N, cus)) {
+    switch (p.part ? 5 : cheapest_tile(kI4Tiles, p.M, p.N, p.K, cus)) {
       case 0: return launch_w_tile<KIND, 1, 1, 4, 3>(p, 1, st);
       case 1: return launch_w_tile<KIND, 1, 2, 4, 3>(p, 1, st);
       case 2: return launch_w_tile<KIND, 2, 2, 2, 3>(p, 1, st);
