@@ -26,10 +26,17 @@
 // 16 u + 4 h + {0..3} and 16 u + 8 + 4 h + {0..3}; the V^T operand reads the same keys (two
 // 8-byte pieces of a V^T row), so both sides agree on which key each product belongs to.
 //
-// LDS (double buffered, one barrier per key block): the K block as 64 rows of hd bf16 with
-// 16-byte chunks XOR-swizzled by the row; V^T as hd rows of 64 keys with 8-byte chunks
-// XOR-swizzled by (row / 2) % 16, written transposed from the loaded V rows.  The next
-// block's global loads are in flight while the current block is computed.
+// LDS (double buffered, one barrier per key block): K and V blocks as 64 rows of hd bf16, as the cache
+// holds them, loaded straight to LDS (buffer_load ... lds) while the previous block is computed.  16-byte
+// chunks are XOR-swizzled by the row so that neither operand's reads conflict: K's are 16-byte reads of 32
+// rows, V's are transposing reads (ds_read_b64_tr_b16: a 16-lane group reads 4 keys x 16 dims and each
+// lane gets one dim's 4 keys).
+//
+// What bounds it: the MFMAs, 96 per wave and block (three terms each way): at 8 x 512 tokens, 32 heads of
+// 128 they take 28 us.  V was transposed by 2-byte LDS stores from registers before (32 conflicting stores
+// per thread and block), and with them the kernel held 404 registers, one wave per SIMD, so nothing ran
+// beside the softmax: 208 us there and 348 us for one 2048-token prompt, 87 and 146 us now, at the same
+// error (2.2e-7 against 64 bits).
 #include <math.h>
 
 #include "../../include/tgm_decoder.h"
@@ -38,8 +45,9 @@
 namespace tgm {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 pa_bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 pa_bf16x4;
 typedef _Float16 pa_f16x4 __attribute__((ext_vector_type(4)));
+typedef short pa_s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) pa_s16x4 pa_lds_s16x4;
 
 constexpr int kPaKeys = 64;      // keys per block
 constexpr int kPaQueries = 128;  // prompt tokens per workgroup (32 per wave)
@@ -60,20 +68,20 @@ __device__ __forceinline__ void pa_split(float (&r)[8], pa_bf16x8 (&t)[kPaTerms]
 
 // Grid (ceil(T / 128), heads, batch), 256 threads.
 template <int HD>
-__global__ void __launch_bounds__(256) dec_prefill_attention(const float* __restrict__ qkv, int T, int H, int HK,
-                                                             const int32_t* __restrict__ pos,
-                                                             const uint16_t* __restrict__ kc,
-                                                             const uint16_t* __restrict__ vc, int max_seq, float scale,
-                                                             void* __restrict__ out, int odt) {
+__global__ void __launch_bounds__(256, 2) dec_prefill_attention(const float* __restrict__ qkv, int T, int H, int HK,
+                                                                const int32_t* __restrict__ pos,
+                                                                const uint16_t* __restrict__ kc,
+                                                                const uint16_t* __restrict__ vc, int max_seq, float scale,
+                                                                void* __restrict__ out, int odt) {
   constexpr int NJ = HD / 16;                         // 16-wide steps of q . k
   constexpr int ND = HD / 32;                         // 32-row tiles of O^T
-  constexpr int KROW = HD * 2, KCH = KROW / 16;       // K block: 64 rows of HD bf16, KCH 16-byte chunks each
-  constexpr int VROW = kPaKeys * 2;                   // V^T block: HD rows of 64 bf16
-  constexpr int KBYTES = kPaKeys * KROW, STAGE = KBYTES + HD * VROW;
-  constexpr int NLD = kPaKeys * KCH / 256;            // 16-byte chunks per thread and block, for K and for V
-  static_assert(NLD * 256 == kPaKeys * KCH, "block loads");
+  constexpr int ROW = HD * 2, CH = ROW / 16;          // a key's row of K or V: CH 16-byte chunks
+  constexpr int BLOCK = kPaKeys * ROW, STAGE = 2 * BLOCK;
+  constexpr int RPI = 1024 / ROW;                     // rows per load instruction
+  constexpr int NLD = kPaKeys / RPI / 4;              // load instructions per wave and block, for K and for V
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * STAGE];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = blockIdx.y, b = blockIdx.z, j = h / (H / HK);
   const int p0 = pos[b];
   const int64_t ld = (int64_t)(H + 2 * HK) * HD;
@@ -91,6 +99,31 @@ __global__ void __launch_bounds__(256) dec_prefill_attention(const float* __rest
   const int wave_minpos = p0 + min(qblk * kPaQueries + wave * 32, T - 1);  // blocks up to it need no mask
   const uint16_t* kbase = kc + ((int64_t)b * HK + j) * max_seq * HD;
   const uint16_t* vbase = vc + ((int64_t)b * HK + j) * max_seq * HD;
+  const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+
+  // Swizzle of a row's chunks.  K: 32 rows at one logical chunk must differ in chunk (or row parity where
+  // two rows share the 64 banks); V: four consecutive rows of 64 consecutive bytes must.
+  auto swz_k = [](int key) { return CH == 16 ? key & 15 : (key >> 1) & 7; };
+  auto swz_v = [](int key) { return CH == 16 ? (key & 3) << 2 : ((key >> 1) & 1) << 2; };
+  // Load offsets: instruction i = wave + 4 q covers rows RPI i ..; lane l fills chunk l % CH of its row.
+  unsigned vok[NLD], vov[NLD];
+#pragma unroll
+  for (int q = 0; q < NLD; ++q) {
+    const int key = RPI * (wave + 4 * q) + lane / CH, ch = lane % CH;
+    vok[q] = (unsigned)(key * ROW + (ch ^ swz_k(key)) * 16);
+    vov[q] = (unsigned)(key * ROW + (ch ^ swz_v(key)) * 16);
+  }
+  auto load_block = [&](int kb) __attribute__((always_inline)) {
+    const int64_t first = (int64_t)kb * kPaKeys;
+    const unsigned bytes = (unsigned)min(kPaKeys, max_seq - (int)first) * ROW;  // keys past the cache read zeros
+    const i32x4v rk = buffer_rsrc(kbase + first * HD, bytes), rv = buffer_rsrc(vbase + first * HD, bytes);
+    const unsigned st = lds_base + (unsigned)((kb & 1) * STAGE + wave * 1024);
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) lds_dma16(rk, st + q * 4096u, vok[q]);
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) lds_dma16(rv, st + (unsigned)BLOCK + q * 4096u, vov[q]);
+  };
+  if (nblocks > 0) load_block(0);
 
   // q terms as the B operand of S^T: lane (query, half) holds q[16 s + 8 half + i] * scale.
   pa_bf16x8 qt[NJ][kPaTerms];
@@ -106,117 +139,88 @@ __global__ void __launch_bounds__(256) dec_prefill_attention(const float* __rest
     }
   }
 
-  u32x4 kreg[NLD], vreg[NLD];
-  auto load_regs = [&](int kb) __attribute__((always_inline)) {
+  // Per-lane LDS offsets.  V: lane i of 16-lane group g reads key + i / 4, dims 16 (g % 2) + 4 (i % 4) .. + 4
+  // of an O^T tile (groups 2 and 3 the keys of lane half 1), and receives dim 16 (g % 2) + i of four keys.
+  const int vi = lane & 15, vg = lane >> 4;
+  const int vkey = 4 * half + (vi >> 2);
+  unsigned voff[ND];
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int c = tid + 256 * i, key = c / KCH, ch = c % KCH;
-      const int kk = min(kb * kPaKeys + key, max_seq - 1);  // keys past the cache are masked
-      kreg[i] = *(const u32x4*)(kbase + (int64_t)kk * HD + ch * 8);
-      vreg[i] = *(const u32x4*)(vbase + (int64_t)kk * HD + ch * 8);
-    }
-  };
-  auto store_lds = [&](int buf) __attribute__((always_inline)) {
-    unsigned char* st = lds + buf * STAGE;
-    unsigned char* vt = st + KBYTES;
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int c = tid + 256 * i, key = c / KCH, ch = c % KCH;
-      *(u32x4*)(st + key * KROW + ((ch ^ (key & (KCH - 1))) * 16)) = kreg[i];
-      const int c8 = key >> 2, sub = (key & 3) * 2;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int d = ch * 8 + e;
-        *(uint16_t*)(vt + d * VROW + ((c8 ^ ((d >> 1) & 15)) * 8) + sub) = (uint16_t)(vreg[i][e >> 1] >> (16 * (e & 1)));
-      }
-    }
-  };
+  for (int dt = 0; dt < ND; ++dt)
+    voff[dt] = (unsigned)(BLOCK + vkey * ROW + ((4 * dt + 2 * (vg & 1) + ((vi & 3) >> 1)) ^ swz_v(vkey)) * 16 + (vi & 1) * 8);
 
   f32x16 O[ND];
 #pragma unroll
   for (int dt = 0; dt < ND; ++dt) O[dt] = f32x16{};
   float m = -INFINITY, l = 0.f;
-  if (nblocks > 0) {
-    load_regs(0);
-    store_lds(0);
-  }
-  __syncthreads();
+#pragma unroll 1
   for (int kb = 0; kb < nblocks; ++kb) {
-    if (kb + 1 < nblocks) load_regs(kb + 1);
+    wait_lds_dma();   // this wave's loads of block kb
+    __syncthreads();  // everybody's; and everybody is done with block kb - 1
+    if (kb + 1 < nblocks) load_block(kb + 1);
+    if (kb * kPaKeys > wave_maxpos) continue;  // uniform over the wave
     const unsigned char* st = lds + (kb & 1) * STAGE;
-    const unsigned char* vt = st + KBYTES;
-    if (kb * kPaKeys <= wave_maxpos) {  // uniform over the wave
-      f32x16 S[2] = {f32x16{}, f32x16{}};
+    f32x16 S[2] = {f32x16{}, f32x16{}};
 #pragma unroll
-      for (int s = 0; s < NJ; ++s)
+    for (int s = 0; s < NJ; ++s)
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-          const int key = kt * 32 + l32;
-          const pa_bf16x8 a = *(const pa_bf16x8*)(st + key * KROW + (((2 * s + half) ^ (key & (KCH - 1))) * 16));
+      for (int kt = 0; kt < 2; ++kt) {
+        const pa_bf16x8 a = *(const pa_bf16x8*)(st + (kt * 32 + l32) * ROW + (((2 * s + half) ^ swz_k(l32)) * 16));
 #pragma unroll
-          for (int t = 0; t < kPaTerms; ++t) S[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qt[s][t], S[kt], 0, 0, 0);
-        }
-      // online softmax of this lane's query over the block (the lane pair l, l ^ 32 holds it)
-      // (scores are in log2 units: q carries scale * log2(e))
-      if (kb * kPaKeys + kPaKeys - 1 > wave_minpos) {  // the block reaches past some query: mask (uniform)
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int key = kb * kPaKeys + kt * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
-            if (key > qpos) S[kt][v] = -INFINITY;
-          }
+        for (int t = 0; t < kPaTerms; ++t) S[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qt[s][t], S[kt], 0, 0, 0);
       }
-      float bm = -INFINITY;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) bm = fmaxf(bm, S[kt][v]);
-      bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
-      const float mn = fmaxf(m, bm);  // finite: block 0 holds key 0 <= qpos
-      float ls = 0.f;
+    // online softmax of this lane's query over the block (the lane pair l, l ^ 32 holds it)
+    // (scores are in log2 units: q carries scale * log2(e))
+    if (kb * kPaKeys + kPaKeys - 1 > wave_minpos) {  // the block reaches past some query: mask (uniform)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const float p = exp2f(S[kt][v] - mn);  // 0 for masked keys
-          S[kt][v] = p;
-          ls += p;
-        }
-      if (__any(mn != m)) {  // some lane's maximum moved: rescale (a wave-uniform branch)
-        const float alpha = m == -INFINITY ? 0.f : exp2f(m - mn);
-        l *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < ND; ++dt)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) O[dt][v] *= alpha;
-      }
-      l += ls;
-      m = mn;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          float r[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) r[i] = S[kt][8 * u + i];
-          pa_bf16x8 pb[kPaTerms];
-          pa_split(r, pb);
-          const int c8 = kt * 8 + u * 4 + half;  // keys 16 u + 4 h .. + 4 of tile kt; + 2: the next 8
-#pragma unroll
-          for (int dt = 0; dt < ND; ++dt) {
-            const int d = dt * 32 + l32;
-            const unsigned char* row = vt + d * VROW;
-            const pa_bf16x4 lo = *(const pa_bf16x4*)(row + ((c8 ^ ((d >> 1) & 15)) * 8));
-            const pa_bf16x4 hi = *(const pa_bf16x4*)(row + (((c8 + 2) ^ ((d >> 1) & 15)) * 8));
-            const pa_bf16x8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-            for (int t = 0; t < kPaTerms; ++t) O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pb[t], O[dt], 0, 0, 0);
-          }
+          const int key = kb * kPaKeys + kt * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
+          if (key > qpos) S[kt][v] = -INFINITY;
         }
     }
-    if (kb + 1 < nblocks) store_lds((kb + 1) & 1);
-    __syncthreads();
+    float bm = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) bm = fmaxf(bm, S[kt][v]);
+    bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+    const float mn = fmaxf(m, bm);  // finite: block 0 holds key 0 <= qpos
+    if (__any(mn != m)) {  // some lane's maximum moved: rescale (a wave-uniform branch)
+      const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) O[dt][v] *= alpha;
+    }
+    m = mn;
+    float ls = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        float r[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          // v_exp_f32: within one unit in the last place; results below 2^-126 become 0, far below the
+          // last place of a sum that holds exp2(0) = 1.  0 for masked keys.
+          r[i] = __builtin_amdgcn_exp2f(S[kt][8 * u + i] - mn);
+          ls += r[i];
+        }
+        pa_bf16x8 pb[kPaTerms];
+        pa_split(r, pb);
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) {  // keys 16 u + 4 h .. + 4 of tile kt, then the ones 8 on
+          const unsigned char* row = st + voff[dt] + (kt * 32 + u * 16) * ROW;
+          const pa_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_s16x4*)row);
+          const pa_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_s16x4*)(row + 8 * ROW));
+          const pa_bf16x8 a = __builtin_bit_cast(pa_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+          for (int t = 0; t < kPaTerms; ++t) O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pb[t], O[dt], 0, 0, 0);
+        }
+      }
+    l += ls;
   }
   l += __shfl_xor(l, 32, 64);
   if (!qvalid) return;
@@ -232,7 +236,7 @@ __global__ void __launch_bounds__(256) dec_prefill_attention(const float* __rest
                                                     (_Float16)(O[dt][4 * g + 2] * inv), (_Float16)(O[dt][4 * g + 3] * inv)};
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) store_from_f32(out, odt, e + i, O[dt][4 * g + i] * inv);
+        for (int i = 0; i < 4; ++i) store_c(out, odt, e + i, O[dt][4 * g + i] * inv);
       }
     }
 }
