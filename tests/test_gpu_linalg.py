@@ -1049,3 +1049,51 @@ def test_gemm_w_stream_parity(dev, fmt):
     for cdt in (torch.float32, torch.bfloat16, torch.float16):
         c = matmul_nt(a, w, scope="ThreadGroup", dtype=cdt)
         assert O.max_rel_err(bf16_np(c)[rows], ref) <= TOL, cdt
+
+
+@pytest.mark.parametrize("fmt,sdt,bs", [("fp4_e2m1", "e8m0", 32), ("fp6_e3m2", "none", 32), ("int4", torch.float16, 128),
+                                        ("uint4", torch.bfloat16, 64)])
+@pytest.mark.parametrize("m", [1, 3, 40])
+def test_repeated_weight_products_equal_first_ones(dev, monkeypatch, fmt, sdt, bs, m):
+    """A remembered plan gives what the general path gives, bit for bit, on other operands of the same key:
+    row strides, unaligned and strided activations, default and explicit dtypes; and every condition that it
+    does not hold (shapes, devices, contiguity, the lowering switch) is still checked."""
+    n, k = 96, 2048
+    rng = np.random.default_rng(m)
+    make = (lambda: make_weight(dev, fmt, n, k, sdt, rng)[0]) if isinstance(sdt, str) else (
+        lambda: int4_weight(dev, fmt, n, k, sdt, bs, rng)[0])
+    xdt = torch.float16 if fmt.endswith("int4") else torch.bfloat16
+    w1, w2 = make(), make()
+    big = torch.randn((m, 2 * k + 64), device=dev).to(xdt)
+    forms = [big[:, :k].contiguous(), big[:, 16:16 + k], big[:, 1:1 + k], big[:, :2 * k:2]]
+    for out in (None, torch.float32, torch.bfloat16):
+        for x in forms:
+            linalg._weight_plans.clear()
+            want = [matmul_nt(x, w1, dtype=out), None]
+            linalg._weight_plans.clear()
+            want[1] = matmul_nt(x, w2, dtype=out)
+            linalg._weight_plans.clear()
+            got = [matmul_nt(x, w, dtype=out) for w in (w1, w1, w2)]
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[0]) and torch.equal(got[2], want[1])
+            assert got[1].dtype is want[0].dtype and got[1].shape == want[0].shape and got[1].is_contiguous()
+            if m == 1:
+                for v in (x[0], big[0, :2 * k:2]):
+                    linalg._weight_plans.clear()
+                    first = matvec(w2, v, out)
+                    linalg._weight_plans.clear()
+                    matvec(w1, v, out)
+                    assert torch.equal(matvec(w2, v, out), first)
+    assert linalg._weight_plans
+    x = forms[0]
+    with pytest.raises(ValueError):
+        matmul_nt(x[:, :k - 32], w1)
+    with pytest.raises((RuntimeError, ValueError)):
+        matmul_nt(x.cpu(), w1)
+    if w1.scales is not None:
+        strided = PackedTensor(w1.data, fmt, (n, k), w1.scales.t().contiguous().t(), bs)
+        assert torch.equal(matmul_nt(x, strided, dtype=torch.float32), matmul_nt(x, w1, dtype=torch.float32))
+    monkeypatch.setattr(linalg, "MI355X_LINALG", 0)
+    linalg.fallbacks.clear()
+    matmul_nt(x, w1, dtype=torch.float32)
+    assert linalg.fallbacks  # the exact-width product, as for a first call
+    linalg.fallbacks.clear()

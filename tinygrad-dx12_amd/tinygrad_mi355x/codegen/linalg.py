@@ -196,6 +196,62 @@ def choose_matrix(weight: PackedTensor | None, activation: torch.Tensor | Packed
     return kernel
 
 
+# Weight products that have run natively, by everything that decides how they run except operand
+# addresses: (format, shape, block size, scale dtype, activation dtype, rows, row stride, output dtype)
+# -> the entry point and its constant arguments.  A repeat skips the checks and choices, which give the
+# same answer for the same key (one GEMV call: 22 -> 6.4 us of host time); alignment and everything
+# else that depends on addresses is the entry point's own check on every call.
+_weight_plans: dict[tuple, tuple] = {}
+_WEIGHT_PLANS_MAX = 4096
+# (operand kinds) -> matrix_intermediate, which depends on nothing else
+_intermediates: dict[tuple, torch.dtype] = {}
+
+
+def _kind(x: torch.Tensor | PackedTensor) -> tuple:
+    return (x.format, None if x.scales is None else x.scales.dtype) if isinstance(x, PackedTensor) else (x.dtype,)
+
+
+def _intermediate(a: torch.Tensor | PackedTensor, b: torch.Tensor | PackedTensor) -> torch.dtype:
+    key = (_kind(a), _kind(b))
+    found = _intermediates.get(key)
+    if found is None:
+        found = _intermediates[key] = matrix_intermediate(a, b)
+    return found
+
+
+def _remember_weight(w: PackedTensor, x: torch.Tensor, out_dtype: torch.dtype) -> None:
+    """Keep the plan of a product that ``_weight_left`` has just run on ``w`` and ``x`` [M, K] as they are."""
+    (n, k), (m, _) = w.shape, x.shape
+    scales, gemv = w.scales, m <= GEMV_MAX_ROWS
+    sdt = None if scales is None else scales.dtype
+    ldx = x.stride(0) if m > 1 else k
+    if len(_weight_plans) >= _WEIGHT_PLANS_MAX:
+        _weight_plans.clear()
+    _weight_plans[(w.format, w.shape, w.block_size, sdt, x.dtype, m, ldx, out_dtype)] = (
+        getattr(K.load_library(), "tgm_gemv" if gemv else "tgm_gemm_w"), gemv, K.FORMAT_IDS[w.format], n, k,
+        -1 if sdt is None else K.dtype_id(sdt), w.block_size, K.dtype_id(x.dtype), m, ldx, K.dtype_id(out_dtype))
+
+
+def _repeat_weight(w: PackedTensor, x: torch.Tensor, m: int, ldx: int, out_dtype: torch.dtype,
+                   shape: tuple[int, ...]) -> torch.Tensor | None:
+    """Run a remembered product, or None when there is no plan for it or any condition that a plan does not
+    hold fails (the general path then decides, and reports)."""
+    data, scales = w.data, w.scales
+    plan = _weight_plans.get((w.format, w.shape, w.block_size, None if scales is None else scales.dtype, x.dtype, m, ldx,
+                              out_dtype))
+    if (plan is None or not MI355X_LINALG or data.get_device() != x.get_device() or not data.is_contiguous()
+            or (scales is not None and not scales.is_contiguous())):
+        return None
+    fn, gemv, fmt, n, k, sdt, bs, xdt, m, ldx, odt = plan
+    y = x.new_empty(shape, dtype=out_dtype)
+    sp = None if scales is None else scales.data_ptr()
+    if gemv:
+        status = fn(data.data_ptr(), fmt, n, k, sp, sdt, bs, x.data_ptr(), xdt, m, ldx, y.data_ptr(), odt, n, K.stream_of(x))
+    else:
+        status = fn(x.data_ptr(), xdt, m, ldx, data.data_ptr(), fmt, n, k, sp, sdt, bs, y.data_ptr(), odt, n, K.stream_of(x))
+    return y if status == K.TGM_OK else None
+
+
 def _weight_left(kernel: MatrixKernel, w: PackedTensor, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     """Y[M, N] = X[M, K] @ deq(W)[N, K]^T through family 1 or 2."""
     n, k = w.shape
@@ -212,6 +268,8 @@ def _weight_left(kernel: MatrixKernel, w: PackedTensor, x: torch.Tensor, out_dty
     if program.kernel is not kernel:
         raise K.UnsupportedKernel(f"{kernel.name}: {m} activation rows belong to {program.kernel.name}")
     program.launch(y.data_ptr(), data.data_ptr(), x.data_ptr(), K.stream_of(x))
+    if data is w.data and scales is w.scales:
+        _remember_weight(w, x, out_dtype)
     return y
 
 
@@ -315,7 +373,7 @@ def matmul(a: torch.Tensor | PackedTensor, b: torch.Tensor | PackedTensor, scope
     device = _validate(a, b, scope, tile)
     if len(a.shape) != 2 or len(b.shape) != 2 or a.shape[1] != b.shape[0]:
         raise ValueError("matrix operands must have compatible rank-two shapes")
-    intermediate = matrix_intermediate(a, b)
+    intermediate = _intermediate(a, b)
     packed = isinstance(a, PackedTensor) or isinstance(b, PackedTensor)
     lhs_dt = intermediate if packed else a.dtype
     rhs_dt = intermediate if packed else b.dtype
@@ -351,10 +409,18 @@ def matmul_nt(a: torch.Tensor | PackedTensor, b: torch.Tensor | PackedTensor, sc
     fused-dequant families; bf16 / f16 / FP8 pairs run the ordinary MFMA GEMM; anything else
     runs ordinary exact compute.
     """
+    if (type(b) is PackedTensor and type(a) is torch.Tensor and scope == "auto" and tile is None and a.dim() == 2
+            and len(b.shape) == 2 and a.shape[1] == b.shape[1] and a.stride(1) == 1):
+        m, k = a.shape
+        if dtype is None:
+            lhs_dt = _intermediate(a, b)
+        y = _repeat_weight(b, a, m, a.stride(0) if m > 1 else k, dtype or _accumulator(lhs_dt, lhs_dt), (m, b.shape[0]))
+        if y is not None:
+            return y
     device = _validate(a, b, scope, tile)
     if len(a.shape) != 2 or len(b.shape) != 2 or a.shape[1] != b.shape[1]:
         raise ValueError("matrix operands must have compatible rank-two shapes")
-    intermediate = matrix_intermediate(a, b)
+    intermediate = _intermediate(a, b)
     packed = isinstance(a, PackedTensor) or isinstance(b, PackedTensor)
     lhs_dt = intermediate if packed else a.dtype
     rhs_dt = intermediate if packed else b.dtype
@@ -408,10 +474,18 @@ def matvec(matrix: torch.Tensor | PackedTensor, vector: torch.Tensor, output_dty
     compute; ``thread=True`` asks for the native GEMV and silently falls back when the
     operands have none, as the reference's thread scope does.
     """
+    if (thread is None and type(matrix) is PackedTensor and type(vector) is torch.Tensor and vector.dim() == 1
+            and len(matrix.shape) == 2 and matrix.shape[1] == vector.shape[0] and vector.stride(0) == 1):
+        n, k = matrix.shape
+        if output_dtype is None:
+            output_dtype = _accumulator(*(_intermediate(matrix, vector),) * 2)
+        y = _repeat_weight(matrix, vector, 1, k, output_dtype, (n,))
+        if y is not None:
+            return y
     device = _device(matrix)
     if len(matrix.shape) != 2 or vector.dim() != 1 or matrix.shape[1] != vector.shape[0] or device != vector.device:
         raise ValueError("matvec expects a matrix and matching vector on one device")
-    intermediate = matrix_intermediate(matrix, vector)
+    intermediate = _intermediate(matrix, vector)
     output_dtype = output_dtype or _accumulator(intermediate, intermediate)
     if thread is None:
         return matmul(matrix, vector.reshape(-1, 1), dtype=output_dtype).reshape(matrix.shape[0])

@@ -41,8 +41,15 @@ def require_device(t: torch.Tensor) -> None:
             "this backend has no CPU implementation")
 
 
+# torch's raw stream handle without the Stream object around it (0.2 against 2.5 us per call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    index = t.get_device()
+    if _raw_stream is None or index < 0:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -140,7 +140,10 @@ def check(name: str, status: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(name, getattr(load_library(), name)(*args))
+    lib = _lib or load_library()  # once loaded it is never replaced
+    status = getattr(lib, name)(*args)
+    if status:
+        check(name, status)
 
 
 def device_arch(ordinal: int) -> str:
