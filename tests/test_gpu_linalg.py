@@ -894,6 +894,42 @@ def test_gemm_mx_fp4_pairs_with_k_a_multiple_of_128(dev, mnk):
     assert O.max_rel_err(bf16_np(c), deq_a @ deq_b.T) <= TOL
 
 
+@pytest.mark.parametrize("mnk", [(20, 100, 128), (33, 1030, 640), (70, 14330, 384), (129, 14300, 896), (250, 14270, 640),
+                                 (515, 14345, 1152)])
+@pytest.mark.parametrize("fa,fb", [("fp6_e2m3", "fp4_e2m1"), ("fp4_e2m1", "fp4_e2m1"), ("fp6_e3m2", "fp6_e2m3"),
+                                   ("fp4_e2m1", "fp6_e3m2")])
+def test_gemm_mx_small_tiles(dev, mnk, fa, fb):
+    """Pairs on the one-tile shapes (32 x 64 up to 128 x 256 as the product grows): ragged edges, K steps that
+    don't fill the last stage of the waves that split K, and a NaN scale (E8M0 0xFF) that begins a row, right
+    behind the last scale of the row before it: it reaches its own row and column only.  Products and their
+    sums' terms are exact in fp32: K terms sum to within K 2^-24 of sum |products|."""
+    m, n, k = mnk
+    rng = np.random.default_rng(m + n)
+    a, deq_a = make_weight(dev, fa, m, k, "e8m0", rng)
+    b, deq_b = make_weight(dev, fb, n, k, "e8m0", rng)
+    a.scales.view(torch.uint8)[m - 1, 0] = 255
+    b.scales.view(torch.uint8)[5, 0] = 255
+    c = matmul_nt(a, b, scope="Wave", dtype=torch.float32).cpu().numpy()
+    assert np.isnan(c[m - 1]).all() and np.isnan(c[:, 5]).all()
+    keep = np.arange(n) != 5
+    got, da, db = c[:m - 1, keep], deq_a[:m - 1], deq_b[keep]
+    assert (np.abs(got - da @ db.T) <= k * 2.0**-24 * (np.abs(da) @ np.abs(db).T)).all()
+
+
+def test_gemm_mx_fp4_stream_of_fewer_tiles_than_compute_units(dev):
+    """115 tiles of 256 x 256, not a multiple of 8: one workgroup each, every output tile sampled."""
+    m, n, k = 1200, 5700, 1024
+    g = torch.Generator(device=dev)
+    g.manual_seed(115)
+    a = quantize_mx(torch.randn((m, k), device=dev, generator=g), "fp4_e2m1")
+    b = quantize_mx(torch.randn((n, k), device=dev, generator=g), "fp4_e2m1")
+    c = matmul_nt(a, b, dtype=torch.float32).cpu().numpy()
+    rng = np.random.default_rng(3)
+    rows, cols = stratified(rng, m, 1), stratified(rng, n, 1)
+    ref = host_dequant_rows(a, rows) @ host_dequant_rows(b, cols).T
+    assert O.max_rel_err(c[np.ix_(rows, cols)], ref) <= TOL
+
+
 def _fp8(dev, shape, dt, rng):
     x = torch.from_numpy(rng.standard_normal(shape).astype(np.float32) * 4).to(dev)
     return x.to(dt)

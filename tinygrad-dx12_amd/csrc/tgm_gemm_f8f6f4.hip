@@ -1,7 +1,8 @@
 // Kernel family 2, scaled-MFMA path for FP4 / FP6 operand pairs: v_mfma_scale_f32_32x32x64_f8f6f4
 // with FP6 (E2M3, E3M2) or FP4 (E2M1) codes on either side, each with E8M0 scales per 32
 // K-elements or unscaled (scale byte 127 = 1.0).  tgm_gemm_mx sends FP4 x FP4 with scales on
-// both sides to its own kernel (tgm_gemm_mx.hip) and every other FP4 / FP6 pair here.
+// both sides to its own kernel (tgm_gemm_mx.hip) and every other FP4 / FP6 pair here.  The kernel
+// below takes large products of short K; the others run on the tiles of tgm_gemm_mx_tile.h.
 //
 // Replaces the reference's collective LinAlg GEMM (alexandreteles/tinygrad-dx12
 // src/tinygrad_dx12/renderer/linalg.py:38-124) for two packed operands.  The reference decodes
@@ -27,57 +28,14 @@
 // one fragment read touches fall in different banks (XOR with (r >> 2) & 3 for 4 columns,
 // rotation by (r >> 3) & 1 for 6).  E8M0 scales arrive four steps at a time (16 bytes per row)
 // into their own double buffer.
-#include "tgm_mfma_common.h"
+#include "tgm_gemm_mx_tile.h"
 
 namespace tgm {
 
-// v_mfma_scale_f32_32x32x64_f8f6f4 operand type codes (cbsz / blgp) of the FP6 / FP4 formats
-constexpr int kOpE2M3 = 2, kOpE3M2 = 3, kOpE2M1 = 4;
-
-template <int T>
-struct F8F6F4 {
-  static constexpr int bits = T <= kOpE3M2 ? 6 : 4;
-  static constexpr int RB = 128 * bits / 8;  // bytes per row and 128-element step
-  static constexpr int C = RB / 16;          // 16-byte columns per row and step
-  static constexpr int L = 4 * bits;         // bytes of one lane's 32 values
-};
-
-template <int C>
-__device__ __forceinline__ int col_phys(int r, int c) {
-  if constexpr (C == 4) return c ^ ((r >> 2) & 3);
-  else return (c + ((r >> 3) & 1)) % 6;
-}
-template <int C>
-__device__ __forceinline__ int col_logical(int r, int pc) {
-  if constexpr (C == 4) return pc ^ ((r >> 2) & 3);
-  else return (pc + 6 - ((r >> 3) & 1)) % 6;
-}
-
-constexpr int kGM = 256, kGN = 128, kGK = 128;  // output tile and K step
+constexpr int kGM = 256, kGN = 128, kGK = kMxK;  // output tile and K step
 constexpr int kGBatchSteps = 4;                 // steps per batch of E8M0 scales
 constexpr int kGBatchRow = kGBatchSteps * kGK / 32;  // scale bytes of one row per batch (16)
 constexpr int kGBatch = (kGM + kGN) * kGBatchRow;    // A and B scales of one batch (6 KB)
-
-// One lane's 32 values of row r (panel at ``panel``) for block kb (0..3) of a step.
-template <int T>
-__device__ __forceinline__ i32x8 read_block(const unsigned char* panel, int r, int kb) {
-  using O = F8F6F4<T>;
-  const unsigned char* row = panel + r * O::RB;
-  i32x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-  if constexpr (O::bits == 4) {
-    const u32x4 q = *(const u32x4*)(row + 16 * col_phys<O::C>(r, kb));
-    v[0] = (int)q[0]; v[1] = (int)q[1]; v[2] = (int)q[2]; v[3] = (int)q[3];
-  } else {  // 24 bytes at 24 kb: three 8-byte pieces, each inside one 16-byte column
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const int b = 24 * kb + 8 * i;
-      const u32x2 q = *(const u32x2*)(row + 16 * col_phys<O::C>(r, b >> 4) + (b & 15));
-      v[2 * i] = (int)q[0];
-      v[2 * i + 1] = (int)q[1];
-    }
-  }
-  return v;
-}
 
 // sa / sb may be null (unscaled operand).  lda / ldb: bytes between rows.
 template <int TA, int TB>
@@ -231,6 +189,12 @@ int launch_f8f6f4(hipStream_t s, int ta, const void* a, int64_t lda, const void*
   if ((sa && (uintptr_t)sa % 4) || (sb && (uintptr_t)sb % 4)) TGM_UNSUPPORTED("%s: scales must be 4-byte aligned", who);
   const unsigned ua = (unsigned)lda, ub = (unsigned)ldb;
   const int im = (int)m, in = (int)n, ik = (int)k;
+  const int shape = mx_tile_shape(ta, tb, m, n, k, false, stream_cu_count(s));
+  if (shape >= 0) {
+    const MxTileArgs p{(const uint8_t*)a, (const uint8_t*)sa, (const uint8_t*)b, (const uint8_t*)sb, c, ldc, ua, ub, im,
+                       in, ik, cdt};
+    return launch_gemm_mx_tile(shape, ta, tb, p, s, who);
+  }
 #define TGM_F8F6F4(A, B)                                                              \
   if (ta == A && tb == B) {                                                           \
     launch_f8f6f4_t<A, B>(s, a, ua, sa, b, ub, sb, im, in, ik, c, cdt, ldc);          \

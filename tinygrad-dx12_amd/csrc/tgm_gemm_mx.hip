@@ -26,10 +26,11 @@
 // LDS in all).  The loads of step s + 2 run while step s + 1's MFMAs do.  Tiles are mapped
 // XCD-aware (tile_of).  For K a multiple of 1024 the same pipeline runs persistently, one
 // workgroup per CU streaming its tiles' steps back to back (gemm_mx_fp4_stream); other K
-// launch one workgroup per tile (gemm_mx_fp4).
+// launch one workgroup per tile (gemm_mx_fp4).  Products whose 256 x 256 tiles leave compute
+// units idle take the smaller tiles of tgm_gemm_mx_tile.h.
 #include <type_traits>
 
-#include "tgm_mfma_common.h"
+#include "tgm_gemm_mx_tile.h"
 
 namespace tgm {
 
@@ -604,9 +605,17 @@ extern "C" int tgm_gemm_mx(const void* a, int a_fmt, const void* a_scales, int64
     TGM_UNSUPPORTED("tgm_gemm_mx: operands must be 16-byte and scales 8-byte aligned");
   const int64_t tiles = ((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
   const int cus = stream_cu_count((hipStream_t)stream);
-  if (k % (kBK * kBatchSteps) == 0 && cus >= 8 && tiles >= 8) {
-    // persistent: one workgroup per CU (a multiple of 8 of them, so each keeps to its XCD's tiles)
-    const int64_t grid = tiles < cus ? tiles / 8 * 8 : cus / 8 * 8;
+  const bool persistent = k % (kBK * kBatchSteps) == 0 && cus >= 8 && tiles >= 8;
+  const int shape = mx_tile_shape(ta, tb, m, n, k, true, cus);
+  if (shape >= 0) {
+    const MxTileArgs p{(const uint8_t*)a, (const uint8_t*)a_scales, (const uint8_t*)b, (const uint8_t*)b_scales, c, ldc,
+                       (unsigned)(k / 2), (unsigned)(k / 2), (int)m, (int)n, (int)k, c_dtype};
+    return launch_gemm_mx_tile(shape, ta, tb, p, (hipStream_t)stream, "tgm_gemm_mx");
+  }
+  if (persistent) {
+    // persistent: one workgroup per CU (a multiple of 8 of them, so each keeps to its XCD's tiles), or per tile where
+    // there are fewer: rounded down to 8, 141 tiles took two rounds (700 x 12000 x 8192 89.5 us, 46 without)
+    const int64_t grid = tiles < cus ? tiles : cus / 8 * 8;
     hipLaunchKernelGGL((gemm_mx_fp4_stream<kWavesM, kWavesN>), dim3((unsigned)grid), dim3(kWavesM * kWavesN * 64), 0,
                        (hipStream_t)stream, (const uint8_t*)a, (const uint8_t*)a_scales, (const uint8_t*)b,
                        (const uint8_t*)b_scales, (int)m, (int)n, (int)k, c, c_dtype, ldc);

@@ -29,7 +29,8 @@ GEMM_W = MatrixKernel("tgm_gemm_w", "ThreadGroup", (256, 128, 128), 512)
 # Family 2: scaled-MFMA GEMM of two packed FP4 / FP6 operands, each with E8M0 block-32 scales or
 # unscaled.  One entry point, two kernels: FP4 x FP4 with both scales and K a multiple of 256
 # runs 256 x 256 tiles with K steps of 256 (GEMM_MX); every other pair, or K a multiple of 128
-# only, runs 256 x 128 tiles with K steps of 128 (GEMM_MX_GENERAL).  ``mx_kernel`` picks.
+# only, runs 256 x 128 tiles with K steps of 128 (GEMM_MX_GENERAL).  ``mx_kernel`` picks.  Where those
+# tiles would leave compute units idle, the entry point itself takes smaller ones.
 GEMM_MX = MatrixKernel("tgm_gemm_mx", "ThreadGroup", (256, 256, 256), 512)
 GEMM_MX_GENERAL = MatrixKernel("tgm_gemm_mx", "ThreadGroup", (256, 128, 128), 512)
 # Family 2: ordinary bf16 x bf16 / f16 x f16 MFMA GEMM (the reference's LinAlg lowering of an
