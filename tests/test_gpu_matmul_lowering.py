@@ -58,6 +58,16 @@ def test_transpose16(dev):
     assert torch.equal(linalg.transpose16(view), view.t())
 
 
+@pytest.mark.parametrize("rows,cols,offset,width", [(8, 8, 0, 8), (64, 256, 0, 256), (72, 1000, 8, 1024), (304, 517, 0, 520),
+                                                    (304, 517, 1, 520), (301, 64, 0, 64), (8, 3, 0, 8), (1, 264, 0, 264)])
+def test_transpose16_blocks(dev, rows, cols, offset, width):
+    """8 x 8 blocks in registers where rows on both sides are 16-byte aligned, ragged edges included; odd row
+    counts, widths and addresses beside them."""
+    x = torch.randint(-30000, 30000, (rows, width + 8), dtype=torch.int16, device=dev)
+    view = x[:, offset:offset + cols]
+    assert torch.equal(linalg.transpose16(view), view.t())
+
+
 def test_ordinary_matmul_eager_gradient_and_replay(dev):
     """The rewritten f16 product keeps its dtype, matches the exact product (rtol/atol 3e-3 as
     the reference's test), gives the right gradients, and replays with changed inputs."""
