@@ -8,7 +8,7 @@ import torch
 
 import decoder_oracle as D
 import packed_oracle as O
-from tinygrad_mi355x.codegen.decomp.mi355x import PackedTensor
+from tinygrad_mi355x.codegen.decomp.mi355x import PackedTensor, quantize_mx
 from tinygrad_mi355x.decoder import Decoder, DecoderConfig, DecoderWeights, random_weights
 from tinygrad_mi355x.runtime import kernels as K
 
@@ -602,7 +602,7 @@ def test_gemv_swiglu_epilogue(dev, nk):
 
 
 # (1000, 16400, 512): 8 x 65 tiles of 128 x 256, at least one round of CUs and K % 512 == 0, so the
-# plain product runs the persistent kernel (gemm_w_stream) and the SwiGLU form gemm_w_mx
+# plain product and the SwiGLU form run the persistent kernel (gemm_w_stream)
 @pytest.mark.parametrize("m,n,k,pad", [(300, 1000, 512, 0), (17, 28672 // 8, 4096, 3), (256, 512, 128, 8),
                                        (1000, 16400, 512, 3)])
 @pytest.mark.parametrize("scaled", [True, False])
@@ -631,6 +631,24 @@ def test_gemm_swiglu_epilogue(dev, m, n, k, pad, scaled):
     g = np64(x) @ O.dequant_f64(O.pack_codes(codes, 4), "fp4_e2m1", (n, k), scales, 32).T
     err = O.max_rel_err(np64(fused[:, :n // 2]), D.silu(g[:, 0::2]) * g[:, 1::2])
     assert err <= 1e-2, err
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+def test_gemm_swiglu_persistent_output_types(dev, dt):
+    """The persistent SwiGLU product in fp32 and f16, ragged in rows and columns, equals the plain product (fp32)
+    followed by tgm_dec_silu_mul bit for bit."""
+    m, n, k = 1001, 16398, 512
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    w = quantize_mx(torch.randn((n, k), device=dev, generator=g), "fp4_e2m1")
+    x = torch.randn((m, k), device=dev, generator=g).to(torch.bfloat16)
+    gu = torch.empty((m, n), dtype=torch.float32, device=dev)
+    fused, sep = (torch.zeros((m, n // 2), dtype=dt, device=dev) for _ in range(2))
+    args = (x.data_ptr(), BF16, m, k, w.data.data_ptr(), 2, n, k, w.scales.data_ptr(), 15, 32)
+    K.call("tgm_gemm_w", *args, gu.data_ptr(), F32, n, stream())
+    K.call("tgm_dec_silu_mul", gu.data_ptr(), m, n // 2, sep.data_ptr(), K.dtype_id(dt), stream())
+    K.call("tgm_gemm_w_swiglu", *args, fused.data_ptr(), K.dtype_id(dt), n // 2, stream())
+    assert torch.equal(fused, sep)
 
 
 @pytest.mark.parametrize("m,n,k", [(8, 28672 // 4, 4096), (2, 1000, 512), (16, 4096, 14336 // 4), (5, 12288, 2048),

@@ -1,6 +1,6 @@
 // Kernel family 2, dequant path: packed FP4 / FP6 weights x bf16 activations on bf16 MFMA, and the
 // choice between the kernels: gemm_w_stream below for at least one round of 128 x 256 tiles,
-// gemm_w_mx for split K and the SwiGLU form, the one-tile kernels of tgm_gemm_w_tile.h for smaller
+// gemm_w_mx for split K, the one-tile kernels of tgm_gemm_w_tile.h for smaller
 // products and for INT4 / UINT4 weights (f16 activations on f16 MFMA).
 //
 // Replaces the reference's collective LinAlg GEMM (alexandreteles/tinygrad-dx12
@@ -86,11 +86,10 @@ __device__ __forceinline__ void decode64(const u32x4* raw, unsigned sbits, bf16x
   }
 }
 
-template <int FMT, bool SCALED, bool SWIGLU = false>
+template <int FMT, bool SCALED>
 __global__ void __launch_bounds__(512) gemm_w_mx(const uint8_t* __restrict__ a, unsigned lda_bytes,
                                                  const uint8_t* __restrict__ w, const uint8_t* __restrict__ sw,
-                                                 int M, int N, int K, void* __restrict__ c, int cdt, int64_t ldc,
-                                                 int kps, float* __restrict__ part) {
+                                                 int M, int N, int K, int kps, float* __restrict__ part) {
   using T = GemmWTraits<FMT>;
   constexpr int FA = 2, FB = 2;
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kWStage + 2 * kWBatch];
@@ -237,13 +236,8 @@ __global__ void __launch_bounds__(512) gemm_w_mx(const uint8_t* __restrict__ a, 
   for (int i = 0; i < FA; ++i)
 #pragma unroll
     for (int j = 0; j < FB; ++j)
-      if (part)
-        store_tile32(acc[i][j], ep, lane, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32, M, N,
-                     part + (int64_t)blockIdx.y * M * N, TGM_F32, N);
-      else if constexpr (SWIGLU)
-        store_tile32_swiglu(acc[i][j], ep, lane, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32, M, N, c, cdt, ldc);
-      else
-        store_tile32(acc[i][j], ep, lane, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32, M, N, c, cdt, ldc);
+      store_tile32(acc[i][j], ep, lane, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32, M, N,
+                   part + (int64_t)blockIdx.y * M * N, TGM_F32, N);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -266,7 +260,8 @@ __global__ void __launch_bounds__(512) gemm_w_mx(const uint8_t* __restrict__ a, 
 //    and writes 16-byte row segments with non-temporal stores.
 // Measured in one process against gemm_w_mx: config 3 (2048 x 11008 x 4096, FP6 E3M2) 156.5 against
 // 171.0 us; with FP4 weights the batch-8 decoder prefill (its down projections 4096 x 4096 x 14336 on
-// this kernel) came out even (15.96 against 15.81 ms).  The SwiGLU form keeps gemm_w_mx.
+// this kernel) came out even (15.96 against 15.81 ms).  The SwiGLU form (FP4, 28672 x 4096 gate and up rows),
+// with the pairs exchanged between lanes in registers: 4096 rows 748 against 769 us, 1024 rows 203 against 218.
 constexpr int kVEpi = 8 * 2048;                                    // one 2 KB epilogue slice per wave
 constexpr int kVLds = 2 * kWStage + 2 * kWBatch + kVEpi;           // 136 KB
 constexpr int kVKMultiple = kWK * kWBatchSteps;                     // K = 512: whole scale batches per tile
@@ -302,7 +297,32 @@ __device__ __forceinline__ void decode_block(const unsigned* raw, int blk, unsig
   }
 }
 
-template <int FMT, bool SCALED>
+// A wave's 32 x 32 block of 16-bit values in its LDS slice to rows r0 .., columns c0 .. of C, 16-byte row segments.
+__device__ __forceinline__ void store_block16(const unsigned short* e16, int lane, int r0, int c0, int M, int N,
+                                              void* c, int64_t ldc) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {  // lane l: row l / 4 + 16 q, columns 8 (l % 4) .. + 8
+    const int r = (lane >> 2) + 16 * q, cc = 8 * (lane & 3);
+    const int row = r0 + r, col = c0 + cc;
+    uint16_t* out = (uint16_t*)c + (int64_t)row * ldc + col;
+    if (row < M) {
+      if (col + 7 < N && ((uintptr_t)out & 15) == 0) {
+        __builtin_nontemporal_store(*(const u32x4*)(e16 + r * 32 + cc), (u32x4*)out);
+      } else {
+#pragma unroll 1
+        for (int e = 0; e < 8 && col + e < N; ++e) out[e] = e16[r * 32 + cc + e];
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int FMT, bool SCALED, bool SWIGLU = false>
 __global__ void __launch_bounds__(512) gemm_w_stream(const uint8_t* __restrict__ a, unsigned lda_bytes,
                                                      const uint8_t* __restrict__ w, const uint8_t* __restrict__ sw,
                                                      int M, int N, int K, void* __restrict__ c, int cdt, int64_t ldc) {
@@ -576,6 +596,36 @@ __global__ void __launch_bounds__(512) gemm_w_stream(const uint8_t* __restrict__
     // + v % 4 of each 32 x 32 tile: columns are weight rows, rows are activation rows).
     const int row0 = tl.mc + wm * 64;
     const int col0 = tl.nc + wn * 64;
+    if constexpr (SWIGLU) {
+      // Even columns are gate, odd ones up: lanes l and l ^ 1 exchange one value of each row pair, the even lane
+      // gets the pair's first row and the odd lane its second.  Both column tiles fill one 32 x 32 block.
+      const int odd = lane & 1, cols = N / 2;
+      unsigned short* e16 = (unsigned short*)ep;
+#pragma unroll
+      for (int i = 0; i < FA; ++i) {
+#pragma unroll
+        for (int j = 0; j < FB; ++j) {
+#pragma unroll
+          for (int v = 0; v < 16; v += 2) {
+            const float x0 = acc[i][j][v], x1 = acc[i][j][v + 1];
+            const float other = __builtin_bit_cast(
+                float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, odd ? x0 : x1), 0xB1, 0xF, 0xF, true));
+            const float g = odd ? other : x0, u = odd ? x1 : other;
+            const float y = g / (1.0f + expf(-g)) * u;
+            const int r = 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3) + odd, cc = 16 * j + ((lane & 31) >> 1);
+            if (cdt == TGM_F32) {
+              const int row = row0 + 32 * i + r, col = col0 / 2 + cc;
+              if (row < M && col < cols) ((float*)c)[(int64_t)row * ldc + col] = y;
+            } else {
+              e16[r * 32 + cc] = cdt == TGM_BF16 ? f32_to_bf16(y) : __builtin_bit_cast(unsigned short, (_Float16)y);
+            }
+          }
+          acc[i][j] = f32x16{};
+        }
+        if (cdt != TGM_F32) store_block16(e16, lane, row0 + 32 * i, col0 / 2, M, cols, c, ldc);
+      }
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < FA; ++i)
 #pragma unroll
@@ -599,26 +649,7 @@ __global__ void __launch_bounds__(512) gemm_w_stream(const uint8_t* __restrict__
             e16[r * 32 + (lane & 31)] = (unsigned short)h;
             e16[(r + 1) * 32 + (lane & 31)] = (unsigned short)(h >> 16);
           }
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {  // lane l: row l / 4 + 16 q, columns 8 (l % 4) .. + 8
-            const int r = (lane >> 2) + 16 * q, cc = 8 * (lane & 3);
-            const int row = row0 + 32 * i + r, col = col0 + 32 * j + cc;
-            uint16_t* out = (uint16_t*)c + (int64_t)row * ldc + col;
-            if (row < M) {
-              if (col + 7 < N && ((uintptr_t)out & 15) == 0) {
-                __builtin_nontemporal_store(*(const u32x4*)(e16 + r * 32 + cc), (u32x4*)out);
-              } else {
-#pragma unroll 1
-                for (int e = 0; e < 8 && col + e < N; ++e) out[e] = e16[r * 32 + cc + e];
-              }
-            }
-          }
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          store_block16(e16, lane, row0 + 32 * i, col0 + 32 * j, M, N, c, ldc);
         }
         acc[i][j] = f32x16{};
       }
@@ -649,27 +680,28 @@ __global__ void __launch_bounds__(256) gemm_split_reduce(const float* __restrict
 template <int FMT, bool SCALED, bool SWIGLU = false>
 int launch_gemm_w(const void* a, int64_t lda, const void* w, const void* scales, int64_t m, int64_t n, int64_t k,
                   void* c, int cdt, int64_t ldc, hipStream_t stream, int splits = 1, float* part = nullptr) {
-  const int64_t tiles = ((m + kWM - 1) / kWM) * ((n + kWN - 1) / kWN);
-  if (!SWIGLU && !part) {  // persistent, one workgroup per CU (a multiple of 8 of them)
+  if (!part) {  // persistent, one workgroup per CU (a multiple of 8 of them)
     const int cus = stream_cu_count(stream);
-    hipLaunchKernelGGL((gemm_w_stream<FMT, SCALED>), dim3((unsigned)(cus / 8 * 8)), dim3(512), 0, stream,
+    hipLaunchKernelGGL((gemm_w_stream<FMT, SCALED, SWIGLU>), dim3((unsigned)(cus / 8 * 8)), dim3(512), 0, stream,
                        (const uint8_t*)a, (unsigned)(lda * 2), (const uint8_t*)w, (const uint8_t*)scales, (int)m,
                        (int)n, (int)k, c, cdt, ldc);
     return launch_status(SWIGLU ? "tgm_gemm_w_swiglu" : "tgm_gemm_w");
   }
-  const int kps = (int)((k / kWK + splits - 1) / splits);
-  hipLaunchKernelGGL((gemm_w_mx<FMT, SCALED, SWIGLU>), dim3((unsigned)tiles, (unsigned)splits), dim3(512), 0, stream,
-                     (const uint8_t*)a, (unsigned)(lda * 2), (const uint8_t*)w, (const uint8_t*)scales, (int)m, (int)n,
-                     (int)k, c, cdt, ldc, kps, part);
-  return launch_status(SWIGLU ? "tgm_gemm_w_swiglu" : "tgm_gemm_w");
+  if constexpr (!SWIGLU) {
+    const int64_t tiles = ((m + kWM - 1) / kWM) * ((n + kWN - 1) / kWN);
+    const int kps = (int)((k / kWK + splits - 1) / splits);
+    hipLaunchKernelGGL((gemm_w_mx<FMT, SCALED>), dim3((unsigned)tiles, (unsigned)splits), dim3(512), 0, stream,
+                       (const uint8_t*)a, (unsigned)(lda * 2), (const uint8_t*)w, (const uint8_t*)scales, (int)m,
+                       (int)n, (int)k, kps, part);
+  }
+  return launch_status("tgm_gemm_w");
 }
 
 }  // namespace tgm
 
 using namespace tgm;
 
-// At least one round of 128 x 256 tiles, and whole scale batches: the persistent kernel's products (and
-// gemm_w_mx's, for the SwiGLU form).  Smaller ones go to the one-tile kernels (figures in tgm_gemm_w_tile.h;
+// At least one round of 128 x 256 tiles, and whole scale batches: the persistent kernel's products.  Smaller ones go to the one-tile kernels (figures in tgm_gemm_w_tile.h;
 // at one round exactly, FP4 2048 x 4096 x 4096: 56.2 us persistent, 57.5 us on one-tile 128 x 256).
 static bool whole_round(int64_t m, int64_t n, int64_t k, int cus) {
   return k % kVKMultiple == 0 && cus >= 8 && ((m + kWM - 1) / kWM) * ((n + kWN - 1) / kWN) >= cus;
