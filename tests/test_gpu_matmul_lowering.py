@@ -68,6 +68,22 @@ def test_transpose16_blocks(dev, rows, cols, offset, width):
     assert torch.equal(linalg.transpose16(view), view.t())
 
 
+@pytest.mark.parametrize("mnk", [(17, 72, 64), (33, 1032, 192), (70, 8200, 320), (257, 4104, 704), (515, 8184, 64),
+                                 (1030, 4104, 192), (1030, 7688, 320)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_dense_small_tiles(dev, mnk, dt):
+    """Single products on the one-tile shapes (32 x 64 up to 128 x 256 as the product grows), ragged edges and K steps
+    that don't fill the last stage of the waves that split K.  Products are exact in fp32: K of them sum to within
+    K 2^-24 of sum |products|.  16-bit results are the fp32 ones rounded."""
+    m, n, k = mnk
+    rng = np.random.default_rng(m + n)
+    a, b = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(dev).to(dt) for s in ((m, k), (k, n)))
+    c = linalg.matmul(a, b, scope="ThreadGroup", dtype=torch.float32)
+    da, db = a.cpu().double().numpy(), b.cpu().double().numpy()
+    assert (np.abs(c.cpu().numpy() - da @ db) <= k * 2.0**-24 * (np.abs(da) @ np.abs(db))).all()
+    assert torch.equal(linalg.matmul(a, b, scope="ThreadGroup", dtype=dt), c.to(dt))
+
+
 def test_ordinary_matmul_eager_gradient_and_replay(dev):
     """The rewritten f16 product keeps its dtype, matches the exact product (rtol/atol 3e-3 as
     the reference's test), gives the right gradients, and replays with changed inputs."""

@@ -13,6 +13,9 @@
 // bind directly, matmul.py:218-226).  Products of two bf16 or two f16 values are exact in
 // fp32; accumulation is fp32 and the output is rounded once.
 //
+// One product of at least a round of 256 x 256 tiles runs the persistent kernel below (K a multiple of
+// 128), smaller ones the tiles of tgm_gemm_dense_tile.h; gemm_dense takes batches and FP8:
+//
 // Workgroup: 128 (M) x 256 (N) output tile, eight waves in 2 x 4 (64 x 64 each, 2 x 2 MFMA
 // tiles).  K advances 64 elements per step: the A panel (128 rows x 128 B) and B panel (256 rows
 // x 128 B) go straight from global memory into a double-buffered LDS stage (buffer_load ... lds,
@@ -21,7 +24,7 @@
 // lane half h.  Loads of step s + 2 run while step s + 1 computes.
 #include <type_traits>
 
-#include "tgm_mfma_common.h"
+#include "tgm_gemm_dense_tile.h"
 
 namespace tgm {
 
@@ -506,6 +509,11 @@ extern "C" int tgm_gemm_dense_batched(const void* a, int a_dtype, int64_t m, int
       hipLaunchKernelGGL((gemm_dense_stream<TGM_F16>), g, dim3(512), 0, st, (const uint8_t*)a, (unsigned)(lda_eff * 2),
                          (const uint8_t*)b, (unsigned)(ldb_eff * 2), (int)m, (int)n, (int)k, c, c_dtype, ldc);
     return launch_status("tgm_gemm_dense");
+  }
+  if (batch == 1) {
+    const DenseTileArgs p{(const uint8_t*)a, (const uint8_t*)b, c, ldc, (unsigned)(lda_eff * 2), (unsigned)(ldb_eff * 2),
+                          (int)m, (int)n, (int)k, c_dtype};
+    return launch_gemm_dense_tile(dense_tile_shape(m, n, k, cus), a_dtype, p, st);
   }
   const int64_t tiles = ((m + kDM - 1) / kDM) * ((n + kDN - 1) / kDN);
   const dim3 grid((unsigned)tiles, (unsigned)batch);

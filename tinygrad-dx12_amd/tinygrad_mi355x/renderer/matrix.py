@@ -34,7 +34,8 @@ GEMM_W = MatrixKernel("tgm_gemm_w", "ThreadGroup", (256, 128, 128), 512)
 GEMM_MX = MatrixKernel("tgm_gemm_mx", "ThreadGroup", (256, 256, 256), 512)
 GEMM_MX_GENERAL = MatrixKernel("tgm_gemm_mx", "ThreadGroup", (256, 128, 128), 512)
 # Family 2: ordinary bf16 x bf16 / f16 x f16 MFMA GEMM (the reference's LinAlg lowering of an
-# ordinary matrix product, codegen/matmul.py:156-246).
+# ordinary matrix product, codegen/matmul.py:156-246).  A single product of few such tiles runs on
+# smaller ones inside the entry point.
 GEMM_DENSE = MatrixKernel("tgm_gemm_dense", "ThreadGroup", (256, 128, 64), 512)
 # The same entry point's persistent kernel for one large product (K a multiple of 128 and at least
 # one round of 256 x 256 tiles on the device's CUs): 256 x 256 tiles, K steps of 64, one workgroup
