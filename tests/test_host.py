@@ -149,6 +149,22 @@ def test_no_cpu_fallback():
         linalg.matmul(PackedTensor(u8([0x21, 0x43]), "uint4", (2, 2)), torch.ones(2, 1))
 
 
+def test_no_cpu_fallback_after_a_native_product(monkeypatch):
+    """A plan left by a product on the GPU doesn't take operands of the same kind that are off it."""
+    w = PackedTensor(torch.zeros(512, dtype=torch.uint8), "fp4_e2m1", (32, 32),
+                     torch.ones((32, 1)).to(torch.float8_e8m0fnu), 32)
+    for m in (1, 4):
+        x = torch.zeros((m, 32), dtype=torch.bfloat16)
+        key = (w.format, w.shape, w.block_size, w.scales.dtype, x.dtype, m, 32, torch.float32)
+        monkeypatch.setitem(linalg._weight_plans, key, (lambda *args: pytest.fail("launched"), True, 2, 32, 32, 15, 32, 12,
+                                                        m, 32, 13))
+        with pytest.raises(RuntimeError, match="no CPU implementation"):
+            linalg.matmul_nt(x, w, dtype=torch.float32)
+        if m == 1:
+            with pytest.raises(RuntimeError, match="no CPU implementation"):
+                linalg.matvec(w, x[0], torch.float32)
+
+
 # ----------------------------------------------------------------------------- registration
 def test_register_is_idempotent_and_opens_no_hardware():
     assert compat.registered() and compat.DEVICES[0] == "MI355X"

@@ -239,7 +239,8 @@ def _repeat_weight(w: PackedTensor, x: torch.Tensor, m: int, ldx: int, out_dtype
     data, scales = w.data, w.scales
     plan = _weight_plans.get((w.format, w.shape, w.block_size, None if scales is None else scales.dtype, x.dtype, m, ldx,
                               out_dtype))
-    if (plan is None or not MI355X_LINALG or data.get_device() != x.get_device() or not data.is_contiguous()
+    index = data.get_device()  # -1 off the GPU: the general path refuses such operands
+    if (plan is None or not MI355X_LINALG or index < 0 or index != x.get_device() or not data.is_contiguous()
             or (scales is not None and not scales.is_contiguous())):
         return None
     fn, gemv, fmt, n, k, sdt, bs, xdt, m, ldx, odt = plan
