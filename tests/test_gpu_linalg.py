@@ -643,6 +643,26 @@ def test_gemm_w_int4_one_hot_is_exact(dev, fmt, bs):
     assert np.array_equal(c, deq[:, cols].T.astype(np.float32))
 
 
+@pytest.mark.parametrize("bs", [32, 64, 128, None])
+@pytest.mark.parametrize("fmt,code", [("int4", 7), ("uint4", 15)])
+def test_gemm_w_int4_sums_in_k_order(dev, fmt, code, bs):
+    """Every scale group size sums K in ascending order, 16 elements at a time.  A row holds 2^15 at k = 0, -2^15 at
+    64 and 2^-10 at one other k: times the code, the small product is below half a last place of the large one.  It
+    is lost between the two, and in the scale group that holds only the second; behind them it stays."""
+    n, k, at = 40, 128, [16, 31, 40, 63, 80, 127]
+    m = 4 * len(at)
+    data = torch.full((n * k // 2,), code * 17, dtype=torch.uint8, device=dev)
+    scales = None if bs is None else torch.ones((n, k // bs), dtype=torch.float16, device=dev)
+    w = PackedTensor(data, fmt, (n, k), scales, bs or 32)
+    a = torch.zeros((m, k), dtype=torch.float16, device=dev)
+    a[:, 0], a[:, 64] = 2.0**15, -2.0**15
+    a[torch.arange(m), torch.tensor(at).repeat(4)] = 2.0**-10
+    c = matmul_nt(a, w, scope="ThreadGroup", dtype=torch.float32).cpu()
+    lost = [x < 64 or (bs in (32, 64) and x // bs == 64 // bs) for x in at]
+    want = torch.tensor([0.0 if gone else code * 2.0**-10 for gone in lost]).repeat(4)
+    assert torch.equal(c, want[:, None].expand(m, n))
+
+
 # one shape per tile of the one-tile kernels (ragged in M and N), step counts that the K groups of a
 # workgroup do not divide, and a single step
 @pytest.mark.parametrize("fmt,sdt,bs", [("fp4_e2m1", "e8m0", 32), ("fp6_e2m3", "e8m0", 32), ("fp6_e3m2", "none", 32),
