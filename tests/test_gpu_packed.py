@@ -225,6 +225,28 @@ def test_quantize_vector_kernel_matches_scalar_kernel(dev, fmt, xdt):
     assert torch.equal(fast.data, slow.data)
 
 
+def test_quantize_fp4_of_2_to_the_35_elements(dev):
+    """2^30 blocks, more than the four lanes a block of the vector kernel's launch can hold: rows at the start,
+    behind 2^31 and 2^32 elements and at the end equal the same rows quantised alone, the zeros between them code 0."""
+    rows, k = 1 << 20, 1 << 15
+    if torch.cuda.mem_get_info(dev)[0] < 100 << 30:
+        pytest.skip("64 GiB of bf16 and 17 GiB of results do not fit")
+    g = torch.Generator(device=dev)
+    g.manual_seed(35)
+    at = torch.tensor([0, 1, (1 << 16) - 1, (1 << 17) + 3, rows // 2, rows - 1], device=dev)
+    some = torch.randn((len(at), k), device=dev, generator=g).to(torch.bfloat16)
+    x = torch.zeros((rows, k), dtype=torch.bfloat16, device=dev)
+    x[at] = some
+    big, small = quantize_mx(x, "fp4_e2m1"), quantize_mx(some, "fp4_e2m1")
+    del x
+    data, scales = big.data.view(rows, k // 2), big.scales.view(torch.uint8)
+    assert torch.equal(data[at], small.data.view(len(at), -1)) and torch.equal(scales[at], small.scales.view(torch.uint8))
+    data[at], scales[at] = 0, 127
+    assert not bool(data.view(torch.int64).any()) and bool((scales == 127).all())
+    del big, data, scales
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("fmt", list(FORMATS))
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("shape,bs", [((64, 1024), 32), ((33, 516), 32), ((257, 40), 24), ((5, 7), 3), ((2049,), 32),

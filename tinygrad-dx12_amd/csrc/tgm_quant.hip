@@ -361,9 +361,11 @@ extern "C" int tgm_quantize_mx(const void* x, int x_dtype, int64_t rows, int64_t
   const int64_t nblk = (k + block_size - 1) / block_size;
   const int64_t total = rows * nblk;
   // Whole 32-element blocks of aligned operands (every contiguous tensor with K a multiple of 32): the
-  // vector kernels.  Other block sizes, ragged last blocks and odd addresses keep the scalar kernel.
+  // vector kernels.  Other block sizes, ragged last blocks and odd addresses keep the scalar kernel, and so
+  // do arrays whose lanes (four a block for FP4, one for FP6) would not fit a launch of 2^32 work items.
+  const int64_t lanes = total * (fmt == TGM_FMT_FP4_E2M1 ? 4 : 1);
   if (block_size == kQBlock && k % kQBlock == 0 && (uintptr_t)x % 16 == 0 &&
-      (uintptr_t)data % (fmt == TGM_FMT_FP4_E2M1 ? 4 : 8) == 0 && total < (1ll << 31)) {
+      (uintptr_t)data % (fmt == TGM_FMT_FP4_E2M1 ? 4 : 8) == 0 && lanes <= (1ll << 32) - 256) {
     const hipStream_t s = (hipStream_t)stream;
     if (x_dtype == TGM_F32) launch_quantize_mx32<TGM_F32>(s, x, total, fmt, data, scales);
     else if (x_dtype == TGM_BF16) launch_quantize_mx32<TGM_BF16>(s, x, total, fmt, data, scales);
