@@ -357,6 +357,28 @@ def test_noalloc_split_k_checks_the_stream_device_before_any_launch():
         K.call("tgm_gemm_w_split_noalloc", 16, 12, 64, 2048, 16, 2, 512, 2048, 16, 15, 32, 16, 13, 512, 4, 0x1000)
 
 
+def _asm_statements(source: str) -> list[list[str]]:
+    """The instructions of every asm statement of a HIP source, as the assembler sees them."""
+    found = []
+    for m in re.finditer(r'\basm\s*(?:volatile)?\s*\(((?:\s*"(?:[^"\\]|\\.)*")+)', source):
+        text = "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', m.group(1)))
+        found.append([i.strip() for i in re.split(r"\\n|\\t|;", text) if i.strip()])
+    return found
+
+
+def test_lds_loads_wait_for_the_scalar_write_of_m0():
+    """gfx9 needs a wait state between a scalar write of M0 and a load to LDS, which takes its address from M0; the
+    compiler fills it in for its own instructions only."""
+    csrc = Path(__file__).resolve().parent.parent / "tinygrad-dx12_amd" / "csrc"
+    loads = 0
+    for path in sorted([*csrc.glob("*.h"), *csrc.glob("*.hip")]):
+        for code in _asm_statements(path.read_text()):
+            for before, after in zip(code, code[1:]):
+                loads += after.endswith(" lds")
+                assert not (re.match(r"s_\w+ m0\b", before) and after.endswith(" lds")), f"{path.name}: {code}"
+    assert loads >= 4  # 2, 4 and 16 bytes a lane, and 16 for some lanes
+
+
 def test_header_enums_match_binding():
     text = HEADER.read_text()
     for name, value in K.FORMAT_IDS.items():

@@ -21,12 +21,16 @@ typedef int i32x4v __attribute__((ext_vector_type(4)));
 // lds_addr + 16 l (4 l).  They are issued as inline assembly so that the compiler does not
 // order later LDS reads of the *other* buffer behind them; completion is awaited
 // explicitly (s_waitcnt vmcnt(0)) before the barrier that publishes a buffer.  M0 is set
-// inside each statement and nothing else in the kernel uses it.
+// inside each statement and nothing else in the kernel uses it.  gfx9 wants one wait state between
+// a scalar write of M0 and an LDS load that reads it (the compiler puts an s_nop 0 there for its own
+// builtin, and nothing inside inline assembly): without it the load may use the previous address.
+// It costs INT4 512 x 6144 x 4096, whose VALU is the bound, 0.9 us of 38.5; FP4 64 x 14336 x 4096, FP6
+// 2048 x 11008 x 4096, the FP4 pair of 4096 x 14336 x 4096 and bf16 4096^3 stay within 0.3 %.
 __device__ __forceinline__ void lds_dma16(i32x4v rsrc, unsigned lds_addr, unsigned voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
 }
 __device__ __forceinline__ void lds_dma4(i32x4v rsrc, unsigned lds_addr, unsigned voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
 }
 __device__ __forceinline__ void wait_lds_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
