@@ -2,6 +2,7 @@
 the no-CPU-fallback rule and the C-ABI library's exports."""
 
 import ctypes
+import importlib.util
 import json
 import re
 import subprocess
@@ -355,6 +356,17 @@ def test_noalloc_split_k_checks_the_stream_device_before_any_launch():
         pytest.skip("a GPU is present: the GPU tests cover the launch path")
     with pytest.raises(ValueError, match="current HIP device|hipStreamGetDevice"):
         K.call("tgm_gemm_w_split_noalloc", 16, 12, 64, 2048, 16, 2, 512, 2048, 16, 15, 32, 16, 13, 512, 4, 0x1000)
+
+
+def test_every_ablation_applies_to_the_kernel_source():
+    """Each variant's edit finds its text in csrc/tgm_gemm_mx.hip and changes it."""
+    path = Path(__file__).resolve().parent.parent / "tinygrad-dx12_amd" / "ablation" / "gemm_mx.py"
+    spec = importlib.util.spec_from_file_location("ablation_gemm_mx", path)
+    ablation = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(ablation)
+    sources = {name: ablation.patched(name) for name in ablation.VARIANTS}
+    assert sources["baseline"] == ablation.SRC.read_text()
+    assert len(set(sources.values())) == len(sources)
 
 
 def _asm_statements(source: str) -> list[list[str]]:

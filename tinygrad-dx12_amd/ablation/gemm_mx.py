@@ -59,7 +59,8 @@ OUT = BUILD / "ablation"
 WORKLOADS = ("fp4_gemm_8192", "fp4_gemm_4096x14336x4096")
 
 STREAM = "gemm_mx_fp4_stream(const uint8_t"
-PERSISTENT = "if (k % (kBK * kBatchSteps) == 0 && cus >= 8 && tiles >= 8) {"
+PERSISTENT = "const bool persistent = k % (kBK * kBatchSteps) == 0 && cus >= 8 && tiles >= 8;"
+LAUNCH_PER_TILE = "const bool persistent = false;"
 # fragment reads in the order the next substep's MFMAs consume them: A0, B0 .. B3, A1 (FA = 2)
 READ_IN_USE_ORDER = "else read_item(fn, rbuf, ru, it == 0 ? 0 : it == FA + FB - 1 ? 1 : it + 1);"
 # fragment and scale reads spread over the first half of a substep's MFMAs, panel loads over the second
@@ -96,8 +97,8 @@ VARIANTS: dict[str, list[tuple[str, str, str]]] = {
     "bf16_mfma": [(STREAM, MX_MFMA, BF16_MFMA)],
     "group_m_4": [("constexpr int kGroupM = 8;", "constexpr int kGroupM = 8;", "constexpr int kGroupM = 4;")],
     "group_m_16": [("constexpr int kGroupM = 8;", "constexpr int kGroupM = 8;", "constexpr int kGroupM = 16;")],
-    "launch_per_tile": [("extern \"C\"", PERSISTENT, "if (false) {")],
-    "waves_2x2": [("extern \"C\"", PERSISTENT, "if (false) {"),
+    "launch_per_tile": [("extern \"C\"", PERSISTENT, LAUNCH_PER_TILE)],
+    "waves_2x2": [("extern \"C\"", PERSISTENT, LAUNCH_PER_TILE),
                   ("extern \"C\"", "hipLaunchKernelGGL((gemm_mx_fp4<kWavesM, kWavesN>), dim3((unsigned)tiles), "
                                    "dim3(kWavesM * kWavesN * 64)",
                    "hipLaunchKernelGGL((gemm_mx_fp4<2, 2>), dim3((unsigned)tiles), dim3(256)")],
