@@ -185,6 +185,18 @@ int tgm_gemm_w_split_noalloc(const void* a, int a_dtype, int64_t m, int64_t lda,
                              int64_t ldc, int64_t splits, void* stream);
 
 /*
+ * What tgm_gemm_w, tgm_gemm_mx and tgm_gemm_dense launch for a product on a device of `cus` compute units
+ * (0: unknown): tile[0] x tile[1] rows and columns of C per workgroup, tile[2] groups of waves that share a
+ * workgroup's K steps, and tile[3] the kernel, 0: a one-tile kernel, chosen by the number of rounds a tile
+ * takes, 1: a kernel of large tiles with one workgroup per tile, 2: a persistent one, a workgroup per compute
+ * unit.  Host code only.  tgm_gemm_w_swiglu takes tgm_gemm_w's tiles.  `block_size` is the INT4 scale group
+ * (0: unscaled), `scaled` whether both packed operands have scales.  No counterpart in the reference.
+ */
+int tgm_gemm_w_tile(int fmt, int64_t block_size, int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* tile);
+int tgm_gemm_mx_tile(int a_fmt, int b_fmt, int scaled, int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* tile);
+int tgm_gemm_dense_tile(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* tile);
+
+/*
  * tgm_gemm_w for FP4 weights whose rows interleave the gate (row 2 i) and up (row 2 i + 1)
  * projections of a SwiGLU block, with the activation in the epilogue:
  *
@@ -208,9 +220,10 @@ int tgm_gemm_w_swiglu(const void* a, int a_dtype, int64_t m, int64_t lda, const 
  *
  * A packed [M, K], B packed [N, K] (FP4 E2M1, FP6 E2M3 or FP6 E3M2), both K contiguous,
  * each with E8M0 scales per 32 K-elements ([M, K/32] / [N, K/32]) or NULL (unscaled:
- * every scale 1).  C (BF16, F16 or F32) row stride ldc; fp32 accumulation.  FP4 x FP4
- * with both scales and K a multiple of 256 runs the 256 x 256-tile FP4 kernel; every
- * other pair needs K a multiple of 128.  INT4 / UINT4 and FP6 E3M2 x E3M2 (whose MFMA
+ * every scale 1).  C (BF16, F16 or F32) row stride ldc; fp32 accumulation.  K must be a
+ * multiple of 128.  FP4 x FP4 with both scales and K a multiple of 256 runs on 256 x 256
+ * tiles and every other pair on 128 x 256 or 256 x 128 ones, or on smaller tiles where those
+ * would leave compute units idle (tgm_gemm_mx_tile).  INT4 / UINT4 and FP6 E3M2 x E3M2 (whose MFMA
  * sums are not exact on gfx950) give TGM_E_UNSUPPORTED.
  */
 int tgm_gemm_mx(const void* a, int a_fmt, const void* a_scales, int64_t m,

@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import packed_oracle as O
+from product_tiles import FP4_PAIR_SIZES, PAIR_SIZES, WEIGHT_SIZES
 from tinygrad_mi355x.codegen import linalg
 from tinygrad_mi355x.codegen.decomp.mi355x import FORMATS, PackedTensor, matmul as decomp_matmul, quantize_mx
 from tinygrad_mi355x.codegen.linalg import matmul, matmul_nt, matvec
@@ -663,13 +664,12 @@ def test_gemm_w_int4_sums_in_k_order(dev, fmt, code, bs):
     assert torch.equal(c, want[:, None].expand(m, n))
 
 
-# one shape per tile of the one-tile kernels (ragged in M and N), step counts that the K groups of a
+# sizes for every tile of the one-tile kernels (ragged in M and N), step counts that the K groups of a
 # workgroup do not divide, and a single step
 @pytest.mark.parametrize("fmt,sdt,bs", [("fp4_e2m1", "e8m0", 32), ("fp6_e2m3", "e8m0", 32), ("fp6_e3m2", "none", 32),
                                         ("int4", torch.float16, 128), ("uint4", torch.bfloat16, 64),
                                         ("int4", torch.float32, 32), ("uint4", torch.float32, 128), ("int4", None, 32)])
-@pytest.mark.parametrize("mnk", [(17, 33, 128), (40, 1000, 640), (70, 4100, 384), (130, 4100, 1152), (200, 6150, 640),
-                                 (500, 6150, 384), (1030, 6150, 256)])
+@pytest.mark.parametrize("mnk", WEIGHT_SIZES)
 def test_gemm_w_one_tile_shapes(dev, fmt, sdt, bs, mnk):
     m, n, k = mnk
     rng = np.random.default_rng(m + n + k + bs)
@@ -686,13 +686,16 @@ def test_gemm_w_one_tile_shapes(dev, fmt, sdt, bs, mnk):
     assert bool(((c.double() - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("fmt", ["fp4_e2m1", "fp6_e2m3", "int4"])
-def test_gemm_w_nan_scales_stay_in_their_row(dev, fmt):
+# 5 steps on two K groups per workgroup; 9, 10 and 11 on four, of which three, two and one have no last step
+@pytest.mark.parametrize("k", [640, 1152, 1280, 1408])
+@pytest.mark.parametrize("fmt,bs", [("fp4_e2m1", 32), ("fp6_e2m3", 32), ("fp6_e3m2", 32), ("int4", 128), ("int4", 64),
+                                    ("int4", 32)])
+def test_gemm_w_nan_scales_stay_in_their_row(dev, fmt, bs, k):
     """K groups past the last step read nothing: a NaN in the next row's first scale stays out."""
-    m, n, k = 20, 96, 640  # 5 steps, 4 K groups per workgroup
+    m, n = 20, 96
     rng = np.random.default_rng(8)
     if fmt == "int4":
-        w, _ = int4_weight(dev, fmt, n, k, torch.float16, 128, rng)
+        w, _ = int4_weight(dev, fmt, n, k, torch.float16, bs, rng)
         w.scales[1::2, 0] = float("nan")
         a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float16)).to(dev)
     else:
@@ -782,7 +785,7 @@ def test_gemm_mx_parity(dev, fa, fb):
 @pytest.mark.parametrize("mnk", [(256, 256, 256), (300, 520, 512), (1000, 777, 768), (40, 1100, 1024), (513, 33, 256)])
 @pytest.mark.parametrize("cdt", [torch.bfloat16, torch.float16, torch.float32])
 def test_gemm_mx_fp4_tiles_and_tails(dev, mnk, cdt):
-    """FP4 x FP4 scaled-MFMA GEMM: whole and ragged 256 x 256 tiles, every output dtype."""
+    """FP4 x FP4 scaled-MFMA GEMM on small tiles, whole and ragged, every output dtype."""
     m, n, k = mnk
     rng = np.random.default_rng(m * 7 + n + k)
     a, deq_a = make_weight(dev, "fp4_e2m1", m, k, "e8m0", rng)
@@ -849,10 +852,11 @@ def test_gemm_mx_fp4_full_size_sampled(dev, mnk):
 @pytest.mark.parametrize("mnk", [(2100, 1300, 1024), (4352, 4352, 2048), (8192, 8448, 1024)])
 @pytest.mark.parametrize("cdt", [torch.bfloat16, torch.float16, torch.float32])
 def test_gemm_mx_fp4_persistent_stream(dev, mnk, cdt):
-    """FP4 x FP4 with K a multiple of 1024 runs the persistent kernel (one workgroup per CU walking
-    several tiles as one stream of K steps).  The shapes give workgroups 1 to 5 tiles, ragged last
-    tiles, tile counts that are and are not multiples of 8 (54, 289, 1056), and K = 1024, where a
-    workgroup moves to its next tile every four steps; every 32 x 32 output tile is sampled."""
+    """FP4 x FP4 with K a multiple of 1024 and many tiles runs the persistent kernel (one workgroup per CU
+    walking several tiles as one stream of K steps).  The two larger shapes give workgroups 1 to 5 tiles,
+    ragged last tiles, tile counts that are and are not multiples of 8 (289, 1056), and K = 1024, where a
+    workgroup moves to its next tile every four steps; the smallest one runs on 128 x 128 tiles.  Every
+    32 x 32 output tile is sampled."""
     m, n, k = mnk
     print(f"persistent FP4 GEMM {m}x{n}x{k} {cdt}", flush=True)
     g = torch.Generator(device=dev)
@@ -874,8 +878,8 @@ MX_PAIRS = [(fa, fb) for fa in ("fp4_e2m1", "fp6_e2m3", "fp6_e3m2") for fb in ("
 @pytest.mark.parametrize("scaled", [(True, True), (True, False), (False, True), (False, False)])
 def test_gemm_mx_every_fp4_fp6_pair(dev, fa, fb, scaled):
     """Every FP4 / FP6 pair, each side E8M0 block-32 scaled or unscaled, on the native scaled MFMA
-    (scope="Wave" raises instead of falling back): ragged 256 x 128 tiles, K = 640 (five steps,
-    two scale batches)."""
+    (scope="Wave" raises instead of falling back): ragged 32 x 64 tiles, K = 640 (five steps on four
+    K groups, two scale batches)."""
     m, n, k = 300, 200, 640
     rng = np.random.default_rng(MX_PAIRS.index((fa, fb)) * 4 + 2 * scaled[0] + scaled[1])
     a, deq_a = make_weight(dev, fa, m, k, "e8m0" if scaled[0] else None, rng)
@@ -914,15 +918,25 @@ def test_gemm_mx_fp4_pairs_with_k_a_multiple_of_128(dev, mnk):
     assert O.max_rel_err(bf16_np(c), deq_a @ deq_b.T) <= TOL
 
 
-@pytest.mark.parametrize("mnk", [(20, 100, 128), (33, 1030, 640), (70, 14330, 384), (129, 14300, 896), (250, 14270, 640),
-                                 (515, 14345, 1152)])
+@pytest.mark.parametrize("mnk", [(70, 14330, 384), (129, 14300, 896), (250, 14270, 640), (515, 14345, 1152), *PAIR_SIZES])
 @pytest.mark.parametrize("fa,fb", [("fp6_e2m3", "fp4_e2m1"), ("fp4_e2m1", "fp4_e2m1"), ("fp6_e3m2", "fp6_e2m3"),
                                    ("fp4_e2m1", "fp6_e3m2")])
 def test_gemm_mx_small_tiles(dev, mnk, fa, fb):
-    """Pairs on the one-tile shapes (32 x 64 up to 128 x 256 as the product grows): ragged edges, K steps that
-    don't fill the last stage of the waves that split K, and a NaN scale (E8M0 0xFF) that begins a row, right
-    behind the last scale of the row before it: it reaches its own row and column only.  Products and their
-    sums' terms are exact in fp32: K terms sum to within K 2^-24 of sum |products|."""
+    """Pairs on every tile (32 x 64 up to 128 x 256 and the 256 x 128 kernel as the product grows): ragged edges,
+    K steps that don't fill the last stage of the waves that split K, and a NaN scale (E8M0 0xFF) that begins a
+    row, right behind the last scale of the row before it: it reaches its own row and column only.  Products and
+    their sums' terms are exact in fp32: K terms sum to within K 2^-24 of sum |products|."""
+    check_pair_with_nan_scales(dev, mnk, fa, fb)
+
+
+@pytest.mark.parametrize("mnk", FP4_PAIR_SIZES)
+def test_gemm_mx_fp4_every_tile(dev, mnk):
+    """FP4 pairs with both scales and K a multiple of 256 on every tile: the small ones, 256 x 256 with one
+    workgroup per tile (K not a multiple of 1024) and the persistent kernel; checked as above."""
+    check_pair_with_nan_scales(dev, mnk, "fp4_e2m1", "fp4_e2m1")
+
+
+def check_pair_with_nan_scales(dev, mnk, fa, fb):
     m, n, k = mnk
     rng = np.random.default_rng(m + n)
     a, deq_a = make_weight(dev, fa, m, k, "e8m0", rng)

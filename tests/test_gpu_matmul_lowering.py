@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import packed_oracle as O
+from product_tiles import DENSE_SIZES
 from tinygrad_mi355x.codegen import linalg
 from tinygrad_mi355x.codegen import matmul as MM
 from tinygrad_mi355x.codegen.decomp.mi355x import FORMATS, PackedTensor
@@ -68,8 +69,7 @@ def test_transpose16_blocks(dev, rows, cols, offset, width):
     assert torch.equal(linalg.transpose16(view), view.t())
 
 
-@pytest.mark.parametrize("mnk", [(17, 72, 64), (33, 1032, 192), (70, 8200, 320), (257, 4104, 704), (515, 8184, 64),
-                                 (1030, 4104, 192), (1030, 7688, 320)])
+@pytest.mark.parametrize("mnk", DENSE_SIZES)
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 def test_dense_small_tiles(dev, mnk, dt):
     """Single products on the one-tile shapes (32 x 64 up to 128 x 256 as the product grows), ragged edges and K steps

@@ -12,6 +12,7 @@ from pathlib import Path
 import pytest
 import torch
 
+import product_tiles as T
 import tinygrad_mi355x
 from tinygrad_mi355x import compat
 from tinygrad_mi355x import dtype as D
@@ -367,6 +368,36 @@ def test_every_ablation_applies_to_the_kernel_source():
     sources = {name: ablation.patched(name) for name in ablation.VARIANTS}
     assert sources["baseline"] == ablation.SRC.read_text()
     assert len(set(sources.values())) == len(sources)
+
+
+def test_product_tests_reach_every_tile():
+    """The sizes of the GPU tests of the weight, pair and dense products run every tile that the entry points have,
+    as these choose for an MI355X."""
+    for fmt, group, name in (("fp4_e2m1", 32, "fp4_e2m1"), ("fp6_e2m3", 32, "fp6"), ("fp6_e3m2", 32, "fp6"),
+                             ("int4", 128, "int4"), ("uint4", 64, "int4"), ("int4", 0, "int4"),
+                             ("int4", 32, "int4 groups of 32")):
+        sizes = T.WEIGHT_SIZES + (T.WEIGHT_PERSISTENT if fmt.startswith("fp") else [])
+        assert {T.weight_tile(fmt, group, *mnk) for mnk in sizes} == T.WEIGHT_TILES[name], fmt
+    for fa, fb in (("fp6_e2m3", "fp4_e2m1"), ("fp4_e2m1", "fp4_e2m1"), ("fp6_e3m2", "fp6_e2m3"), ("fp4_e2m1", "fp6_e3m2")):
+        sixes = fa.startswith("fp6") + fb.startswith("fp6")
+        assert {T.pair_tile(fa, fb, True, *mnk) for mnk in T.PAIR_SIZES} == T.PAIR_TILES[sixes], (fa, fb)
+    assert {T.pair_tile("fp4_e2m1", "fp4_e2m1", True, *mnk) for mnk in T.FP4_PAIR_SIZES} == T.FP4_PAIR_TILES
+    assert {T.dense_tile(*mnk) for mnk in T.DENSE_SIZES + T.DENSE_PERSISTENT} == T.DENSE_TILES
+
+
+@pytest.mark.parametrize("fa,fb,mnk,tile", [
+    # FP4 pairs with K not a multiple of 256: 256 x 128 tiles run two to a compute unit (us on it, on 128 x 256 tiles)
+    ("fp4_e2m1", "fp4_e2m1", (700, 14336, 640), (256, 128)),  # 13.4, 22.2
+    ("fp4_e2m1", "fp4_e2m1", (3000, 14336, 2432), (256, 128)),  # 80.2, 107.6
+    ("fp4_e2m1", "fp4_e2m1", (2048, 14336, 1152), (256, 128)),  # 34.0, 44.9
+    # one 6-bit operand: 256 x 128 for short K, 128 x 256 for long K
+    ("fp6_e2m3", "fp4_e2m1", (4096, 9842, 1152), (256, 128)),  # 149.0, 161.4
+    ("fp4_e2m1", "fp6_e3m2", (4096, 14336, 1152), (256, 128)),  # 90.7, 100.4
+    ("fp6_e2m3", "fp4_e2m1", (2048, 4096, 7552), (128, 256)),  # 66.2, 58.3
+    ("fp6_e2m3", "fp6_e3m2", (700, 14336, 640), (256, 128)),  # 23.5, 29.9
+])
+def test_pairs_take_the_tile_that_measures_faster(fa, fb, mnk, tile):
+    assert T.pair_tile(fa, fb, True, *mnk)[:2] == tile
 
 
 def _asm_statements(source: str) -> list[list[str]]:

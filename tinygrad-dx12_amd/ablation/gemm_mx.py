@@ -59,7 +59,7 @@ OUT = BUILD / "ablation"
 WORKLOADS = ("fp4_gemm_8192", "fp4_gemm_4096x14336x4096")
 
 STREAM = "gemm_mx_fp4_stream(const uint8_t"
-PERSISTENT = "const bool persistent = k % (kBK * kBatchSteps) == 0 && cus >= 8 && tiles >= 8;"
+PERSISTENT = "const bool persistent = streams(m, n, k, cus);"
 LAUNCH_PER_TILE = "const bool persistent = false;"
 # fragment reads in the order the next substep's MFMAs consume them: A0, B0 .. B3, A1 (FA = 2)
 READ_IN_USE_ORDER = "else read_item(fn, rbuf, ru, it == 0 ? 0 : it == FA + FB - 1 ? 1 : it + 1);"

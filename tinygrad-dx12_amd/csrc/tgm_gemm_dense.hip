@@ -470,6 +470,20 @@ __global__ void __launch_bounds__(256) transpose16_blocks(const uint16_t* __rest
 
 using namespace tgm;
 
+// One product of at least a round of 256 x 256 tiles: the persistent kernel's.
+static bool streams(int64_t m, int64_t n, int64_t k, int cus) {
+  return k % 128 == 0 && cus >= 8 && ((m + kSB - 1) / kSB) * ((n + kSB - 1) / kSB) >= cus;
+}
+
+extern "C" int tgm_gemm_dense_tile(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* tile) {
+  clear_error();
+  TGM_CHECK_ARG(tile && m > 0 && n > 0 && k > 0 && k % kDK == 0 && cus >= 0 && cus < (1 << 20), "invalid gemm sizes");
+  if (streams(m, n, k, (int)cus)) return tell_tile({kSB, kSB, 1, kPersistent}, tile);
+  TileChoice t;
+  dense_tile_shape(m, n, k, (int)cus, &t);
+  return tell_tile(t, tile);
+}
+
 extern "C" int tgm_gemm_dense_batched(const void* a, int a_dtype, int64_t m, int64_t lda, int64_t stride_a,
                                       const void* b, int b_dtype, int64_t n, int64_t ldb, int64_t stride_b,
                                       int64_t b_group, int64_t k, void* c, int c_dtype, int64_t ldc, int64_t stride_c,
@@ -497,9 +511,8 @@ extern "C" int tgm_gemm_dense_batched(const void* a, int a_dtype, int64_t m, int
       (n - 1) * ldb_eff * 2 + k * 2 >= (1ll << 32) || batch > 65535)
     TGM_UNSUPPORTED("tgm_gemm_dense: operands must be under 4 GiB (32-bit offsets), at most 65535 batches");
   const hipStream_t st = (hipStream_t)stream;
-  const int64_t tiles_s = ((m + kSB - 1) / kSB) * ((n + kSB - 1) / kSB);
   const int cus = stream_cu_count(st);
-  if (batch == 1 && k % 128 == 0 && cus >= 8 && tiles_s >= cus) {
+  if (batch == 1 && streams(m, n, k, cus)) {
     // one large product: persistent, one workgroup per CU (a multiple of 8 of them)
     const dim3 g((unsigned)(cus / 8 * 8));
     if (a_dtype == TGM_BF16)

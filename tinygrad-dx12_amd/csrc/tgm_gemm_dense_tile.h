@@ -200,8 +200,9 @@ int launch_dense_tile(const DenseTileArgs& p, hipStream_t s) {
   return launch_status("tgm_gemm_dense");
 }
 
-// The tile shape for a product.  cus: compute units of the stream's device (0 if unknown).
-int dense_tile_shape(int64_t m, int64_t n, int64_t k, int cus);
+// The tile shape for a product, and the tile itself in *tile.  cus: compute units of the stream's device (0 if
+// unknown).
+int dense_tile_shape(int64_t m, int64_t n, int64_t k, int cus, TileChoice* tile = nullptr);
 int launch_gemm_dense_tile(int shape, int dtype, const DenseTileArgs& p, hipStream_t s);
 
 }  // namespace tgm

@@ -4,12 +4,20 @@
 namespace tgm {
 
 // us at K = 4096 (M and N varied) for the shapes in launch_dtype's order; the ratios hold from K = 512 to 8192, so no
-// shape asks for a longest or shortest K.
-static constexpr TileCost kDenseTiles[] = {{32, 64, 1, 10.2f, 13.2f, 21.0f, 24.0f},   {64, 64, 1, 12.5f, 16.2f, 28.0f, 30.7f},
-                                           {64, 128, 1, 17.0f, 24.0f, 39.0f, 43.2f},  {128, 128, 1, 26.5f, 34.8f, 60.0f, 67.5f},
-                                           {128, 256, 1, 43.3f, 62.0f, 98.0f, 118.0f}};
+// shape asks for a longest or shortest K.  Below, the smaller tiles' larger share that does not grow with K counts
+// (700 x 14336 x 128: 16.0 us on 128 x 128, 14.5 on 128 x 256).
+static constexpr TileCost kDenseTiles[] = {{32, 64, 1, 10.2f, 13.2f, 21.0f, 24.0f, 0.15f},
+                                           {64, 64, 1, 12.5f, 16.2f, 28.0f, 30.7f, 0.15f},
+                                           {64, 128, 1, 17.0f, 24.0f, 39.0f, 43.2f, 0.15f},
+                                           {128, 128, 1, 26.5f, 34.8f, 60.0f, 67.5f, 0.15f},
+                                           {128, 256, 1, 43.3f, 62.0f, 98.0f, 118.0f, 0.11f}};
+static constexpr int kGroups[] = {4, 2, 2, 1, 1};  // launch_dtype's K groups by shape
 
-int dense_tile_shape(int64_t m, int64_t n, int64_t k, int cus) { return cheapest_tile(kDenseTiles, m, n, k, cus); }
+int dense_tile_shape(int64_t m, int64_t n, int64_t k, int cus, TileChoice* tile) {
+  const int i = cheapest_tile(kDenseTiles, m, n, k, cus);
+  if (tile) *tile = {kDenseTiles[i].bm, kDenseTiles[i].bn, kGroups[i], kOneTile};
+  return i;
+}
 
 template <int T16>
 static int launch_dtype(int shape, const DenseTileArgs& p, hipStream_t s) {

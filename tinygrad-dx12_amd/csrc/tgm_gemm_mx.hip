@@ -274,8 +274,8 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mx_fp4(const uint8_t* __res
 
 // ---------------------------------------------------------------------------------------------
 // Persistent form for K a multiple of 1024 (kBatchSteps steps of 256): one workgroup per CU walks
-// the tiles blockIdx.x, blockIdx.x + G, ... (G = gridDim.x, a multiple of 8, so a workgroup's tiles
-// stay on its XCD's contiguous range of tile_of) as one stream of K steps.  The step pipeline of
+// the tiles blockIdx.x, blockIdx.x + G, ... (G = gridDim.x: every tile has its own workgroup, or G is a
+// multiple of 8, so that a workgroup's tiles stay on its XCD's range of tile_of) as one stream of K steps.  The step pipeline of
 // gemm_mx_fp4 runs across tile boundaries unchanged: the loads of the next tile's first two
 // steps are issued during the current tile's last two, so a tile starts with its operands in LDS
 // instead of waiting for them, and no workgroup is launched per tile.  At a tile's end the
@@ -580,6 +580,26 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_mx_fp4_stream(const uint8_t
 
 using namespace tgm;
 
+static int64_t large_tiles(int64_t m, int64_t n) { return ((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN); }
+// The 256 x 256 kernel that walks its tiles takes whole scale batches.
+static bool streams(int64_t m, int64_t n, int64_t k, int cus) {
+  return k % (kBK * kBatchSteps) == 0 && cus >= 8 && large_tiles(m, n) >= 8;
+}
+
+extern "C" int tgm_gemm_mx_tile(int a_fmt, int b_fmt, int scaled, int64_t m, int64_t n, int64_t k, int64_t cus,
+                                int64_t* tile) {
+  clear_error();
+  TGM_CHECK_ARG(valid_format(a_fmt) && valid_format(b_fmt) && tile, "unknown packed format, or no result");
+  TGM_CHECK_ARG(m > 0 && n > 0 && k > 0 && k % kMxK == 0 && cus >= 0 && cus < (1 << 20), "invalid gemm sizes");
+  const int ta = f8f6f4_code_of_format(a_fmt), tb = f8f6f4_code_of_format(b_fmt);
+  if (ta < 0 || tb < 0 || (ta == kOpE3M2 && tb == kOpE3M2))
+    TGM_UNSUPPORTED("tgm_gemm_mx_tile: no scaled-MFMA kernel for these formats");
+  const bool big = ta == kOpE2M1 && tb == kOpE2M1 && scaled && k % kBK == 0;
+  TileChoice t;
+  if (mx_tile_shape(ta, tb, m, n, k, big, (int)cus, &t) < 0 && big && streams(m, n, k, (int)cus)) t.kernel = kPersistent;
+  return tell_tile(t, tile);
+}
+
 extern "C" int tgm_gemm_mx(const void* a, int a_fmt, const void* a_scales, int64_t m, const void* b, int b_fmt,
                            const void* b_scales, int64_t n, int64_t k, void* c, int c_dtype, int64_t ldc,
                            void* stream) {
@@ -603,9 +623,9 @@ extern "C" int tgm_gemm_mx(const void* a, int a_fmt, const void* a_scales, int64
     TGM_UNSUPPORTED("tgm_gemm_mx: operands must be under 4 GiB (32-bit offsets)");
   if ((uintptr_t)a % 16 || (uintptr_t)b % 16 || (uintptr_t)a_scales % 8 || (uintptr_t)b_scales % 8)
     TGM_UNSUPPORTED("tgm_gemm_mx: operands must be 16-byte and scales 8-byte aligned");
-  const int64_t tiles = ((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
+  const int64_t tiles = large_tiles(m, n);
   const int cus = stream_cu_count((hipStream_t)stream);
-  const bool persistent = k % (kBK * kBatchSteps) == 0 && cus >= 8 && tiles >= 8;
+  const bool persistent = streams(m, n, k, cus);
   const int shape = mx_tile_shape(ta, tb, m, n, k, true, cus);
   if (shape >= 0) {
     const MxTileArgs p{(const uint8_t*)a, (const uint8_t*)a_scales, (const uint8_t*)b, (const uint8_t*)b_scales, c, ldc,

@@ -263,9 +263,10 @@ int launch_mx_tile(const MxTileArgs& p, hipStream_t s, const char* who) {
   return launch_status(who);
 }
 
-// The tile shape for a product, -1 for the 256-row kernels.  fp4_big: the 256 x 256 FP4 kernels take the operands
-// (else gemm_f8f6f4 does).  cus: compute units of the stream's device (0 if unknown).
-int mx_tile_shape(int ta, int tb, int64_t m, int64_t n, int64_t k, bool fp4_big, int cus);
+// The tile shape for a product, -1 for the large-tile kernels.  fp4_big: the 256 x 256 FP4 kernels take the
+// operands (else gemm_f8f6f4 does).  cus: compute units of the stream's device (0 if unknown).  The tile that
+// runs goes to *tile.
+int mx_tile_shape(int ta, int tb, int64_t m, int64_t n, int64_t k, bool fp4_big, int cus, TileChoice* tile = nullptr);
 int launch_gemm_mx_tile(int shape, int ta, int tb, const MxTileArgs& p, hipStream_t s, const char* who);
 
 }  // namespace tgm

@@ -701,8 +701,9 @@ int launch_gemm_w(const void* a, int64_t lda, const void* w, const void* scales,
 
 using namespace tgm;
 
-// At least one round of 128 x 256 tiles, and whole scale batches: the persistent kernel's products.  Smaller ones go to the one-tile kernels (figures in tgm_gemm_w_tile.h;
-// at one round exactly, FP4 2048 x 4096 x 4096: 56.2 us persistent, 57.5 us on one-tile 128 x 256).
+// At least one round of 128 x 256 tiles, and whole scale batches: the persistent kernel's products.  Smaller
+// ones go to the one-tile kernels (figures in tgm_gemm_w_tile.h; at one round exactly, FP4 2048 x 4096 x 4096:
+// 56.2 us persistent, 57.5 us on one-tile 128 x 256).
 static bool whole_round(int64_t m, int64_t n, int64_t k, int cus) {
   return k % kVKMultiple == 0 && cus >= 8 && ((m + kWM - 1) / kWM) * ((n + kWN - 1) / kWN) >= cus;
 }
@@ -767,6 +768,15 @@ static int gemm_w_impl(const void* a, int a_dtype, int64_t m, int64_t lda, const
     case TGM_FMT_FP6_E3M2 * 2 + 1: return launch_gemm_w<TGM_FMT_FP6_E3M2, true>(a, lda_eff, w, scales, m, n, k, c, c_dtype, ldc, st, splits, part);
     default: return launch_gemm_w<TGM_FMT_FP6_E3M2, false>(a, lda_eff, w, scales, m, n, k, c, c_dtype, ldc, st, splits, part);
   }
+}
+
+extern "C" int tgm_gemm_w_tile(int fmt, int64_t block_size, int64_t m, int64_t n, int64_t k, int64_t cus, int64_t* tile) {
+  clear_error();
+  TGM_CHECK_ARG(valid_format(fmt) && tile, "unknown packed format %d or no result", fmt);
+  TGM_CHECK_ARG(m > 0 && n > 0 && k > 0 && k % kWK == 0 && cus >= 0 && cus < (1 << 20), "invalid gemm sizes");
+  if (fmt == TGM_FMT_INT4 || fmt == TGM_FMT_UINT4) return tell_tile(w_tile_i4(block_size, m, n, k, (int)cus), tile);
+  if (whole_round(m, n, k, (int)cus)) return tell_tile({kWM, kWN, 1, kPersistent}, tile);
+  return tell_tile(w_tile_mx(fmt, m, n, k, (int)cus), tile);
 }
 
 extern "C" int tgm_gemm_w(const void* a, int a_dtype, int64_t m, int64_t lda, const void* w, int fmt, int64_t n,

@@ -438,21 +438,22 @@ int launch_w_tile(const WTileArgs& p, int splits, hipStream_t stream) {
 }
 
 // The choice of tile.  A shape's time is that of the rounds of workgroups it takes: `lo` us for a first
-// round of few workgroups and `hi` for one on every compute unit (measured at K = 4096; the ratios, which
-// decide, hold for K = 1024 to 14336), and lo2 .. hi2 for two (less than twice where two workgroups fit a
-// compute unit's LDS).  The smallest estimate wins, so a product takes the smallest tile that still gives
-// every compute unit one workgroup, and larger tiles, which read less per MFMA, as it grows.
+// round of few workgroups and `hi` for one on every compute unit (measured at K = 4096), and lo2 .. hi2 for
+// two (less than twice where two workgroups fit a compute unit's LDS).  `fixed` is the share of that time
+// that does not grow with K (launch, prologue, epilogue), where shapes that compete differ in it; the others
+// leave it 0, and only their ratios count.  The smallest estimate wins, so a product takes the smallest tile
+// that still gives every compute unit one workgroup, and larger tiles, which read less per MFMA, as it grows.
 // Shapes that split K over wk waves want two K steps for each; shorter products go to the others.
 struct TileCost {
   int bm, bn, wk;
-  float lo, hi, lo2, hi2;
+  float lo, hi, lo2, hi2, fixed;
 };
-inline float tile_estimate(const TileCost& t, int64_t m, int64_t n, int64_t cus) {
+inline float tile_estimate(const TileCost& t, int64_t m, int64_t n, int64_t k, int64_t cus) {
   const int64_t w = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
   const int64_t pairs = w / (2 * cus), rest = w - pairs * 2 * cus;
   const float f = (float)(rest % cus ? rest % cus : cus) / (float)cus;
   const float tail = rest == 0 ? 0.f : rest <= cus ? t.lo + (t.hi - t.lo) * f : t.lo2 + (t.hi2 - t.lo2) * f;
-  return (float)pairs * t.hi2 + tail;
+  return ((float)pairs * t.hi2 + tail) * (t.fixed + (1.f - t.fixed) * (float)k / 4096.f);
 }
 template <int COUNT>
 int cheapest_tile(const TileCost (&table)[COUNT], int64_t m, int64_t n, int64_t k, int cus) {
@@ -460,7 +461,7 @@ int cheapest_tile(const TileCost (&table)[COUNT], int64_t m, int64_t n, int64_t 
   float least = 0.f;
   for (int i = 0; i < COUNT; ++i) {
     if (table[i].wk > 1 && k / kWtK < 2 * table[i].wk) continue;
-    const float e = tile_estimate(table[i], m, n, cus > 0 ? cus : 256);
+    const float e = tile_estimate(table[i], m, n, k, cus > 0 ? cus : 256);
     if (best < 0 || e < least) {
       best = i;
       least = e;
@@ -469,9 +470,25 @@ int cheapest_tile(const TileCost (&table)[COUNT], int64_t m, int64_t n, int64_t 
   return best;
 }
 
+// What an entry point launches for a product (the tgm_*_tile queries): rows and columns of C per workgroup,
+// wave groups that share its K steps, and the kind of kernel.
+constexpr int kOneTile = 0, kLargeTile = 1, kPersistent = 2;
+struct TileChoice {
+  int rows, cols, k_groups, kernel;
+};
+inline int tell_tile(const TileChoice& t, int64_t* tile) {
+  tile[0] = t.rows;
+  tile[1] = t.cols;
+  tile[2] = t.k_groups;
+  tile[3] = t.kernel;
+  return TGM_OK;
+}
+
 // One-tile products by format; tgm_gemm_w_tile_mx.hip and tgm_gemm_w_tile_i4.hip.  cus: compute units of
 // the stream's device (0 if unknown).
 int launch_gemm_w_tile_mx(const WTileArgs& p, int fmt, int cus, hipStream_t stream);
 int launch_gemm_w_tile_i4(const WTileArgs& p, int64_t block_size, int splits, int cus, hipStream_t stream);
+TileChoice w_tile_mx(int fmt, int64_t m, int64_t n, int64_t k, int cus);
+TileChoice w_tile_i4(int64_t group, int64_t m, int64_t n, int64_t k, int cus);
 
 }  // namespace tgm

@@ -12,6 +12,12 @@ static constexpr TileCost kI4Tiles32[] = {
     {32, 32, 4, 12.2f, 13.8f, 24.4f, 25.5f},  {64, 32, 4, 16.7f, 19.9f, 34.7f, 35.8f},  {64, 64, 2, 23.9f, 26.3f, 48.5f, 49.0f},
     {64, 128, 2, 28.6f, 36.2f, 67.0f, 70.0f}, {128, 256, 1, 73.0f, 88.0f, 153.0f, 160.0f}};
 
+TileChoice w_tile_i4(int64_t group, int64_t m, int64_t n, int64_t k, int cus) {
+  const TileCost& t = group == 32 ? kI4Tiles32[cheapest_tile(kI4Tiles32, m, n, k, cus)]
+                                  : kI4Tiles[cheapest_tile(kI4Tiles, m, n, k, cus)];
+  return {t.bm, t.bn, t.wk, kOneTile};
+}
+
 template <int KIND>
 static int launch_kind(const WTileArgs& p, int splits, int cus, hipStream_t st) {
   // split K keeps the largest tile: its callers split products whose 128 x 256 tiles are few
