@@ -61,7 +61,7 @@ gemm_dense_tile(DenseTileArgs p) {
   const int wk = wave / T::kW, w = wave % T::kW, wm = w / WN, wn = w % WN;
   const int tiles_m = (p.M + T::kBM - 1) / T::kBM, tiles_n = (p.N + T::kBN - 1) / T::kBN;
   int tm, tn;
-  tile_of(blockIdx.x, tiles_m, tiles_n, 8, tm, tn);
+  tile_of_ranges(blockIdx.x, p.K, tiles_m, tiles_n, 8, tm, tn);
   const int m0 = tm * T::kBM, n0 = tn * T::kBN;
   const int nsteps = p.K / kDtK, nstages = (nsteps + WK - 1) / WK;
   const i32x4v ra = buffer_rsrc(p.a, (unsigned)(p.M - 1) * p.lda + (unsigned)p.K * 2u);

@@ -85,7 +85,7 @@ gemm_mx_tile(MxTileArgs p) {
   const int wk = wave / T::kW, w = wave % T::kW, wm = w / WN, wn = w % WN;
   const int tiles_m = (p.M + T::kBM - 1) / T::kBM, tiles_n = (p.N + T::kBN - 1) / T::kBN;
   int tm, tn;
-  tile_of(blockIdx.x, tiles_m, tiles_n, 8, tm, tn);
+  tile_of_ranges(blockIdx.x, p.K, tiles_m, tiles_n, 8, tm, tn);
   const int m0 = tm * T::kBM, n0 = tn * T::kBN;
   const int nsteps = p.K / kMxK, nstages = (nsteps + WK - 1) / WK;
   const unsigned kblk = (unsigned)(p.K / 32);

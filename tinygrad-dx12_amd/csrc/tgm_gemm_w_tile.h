@@ -185,7 +185,7 @@ gemm_w_tile(WTileArgs p) {
   const int wn = wave % WN, wk = wave / WN;
   const int tiles_m = (p.M + T::kBM - 1) / T::kBM, tiles_n = (p.N + T::kBN - 1) / T::kBN;
   int tm, tn;
-  tile_of(blockIdx.x, tiles_m, tiles_n, 8, tm, tn);
+  tile_of_ranges(blockIdx.x, p.K, tiles_m, tiles_n, 8, tm, tn);
   const int m0 = tm * T::kBM, n0 = tn * T::kBN;
   // split K (WK == 1 shapes only): steps s_begin .. of this workgroup
   const int s_begin = WK == 1 && p.part ? (int)blockIdx.y * p.steps_per_split : 0;

@@ -44,9 +44,7 @@ __device__ __forceinline__ i32x4v buffer_rsrc(const void* p, unsigned bytes) {
 // to give each XCD a contiguous range of tiles (when the count divides by 8), walked in
 // groups of ``group_m`` row panels so that concurrently running tiles share operand panels
 // in that XCD's L2.
-__device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
-  const int ntiles = tiles_m * tiles_n;
-  if (ntiles % 8 == 0) pid = (pid % 8) * (ntiles / 8) + pid / 8;  // contiguous range per XCD
+__device__ __forceinline__ void tile_at(int pid, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
   const int per_group = group_m * tiles_n;
   const int group = pid / per_group;
   const int first_m = group * group_m;
@@ -54,6 +52,25 @@ __device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int g
   const int in_group = pid - group * per_group;
   tm = first_m + in_group % gsize;
   tn = in_group / gsize;
+}
+__device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
+  const int ntiles = tiles_m * tiles_n;
+  if (ntiles % 8 == 0) pid = (pid % 8) * (ntiles / 8) + pid / 8;  // contiguous range per XCD
+  tile_at(pid, tiles_m, tiles_n, group_m, tm, tn);
+}
+// The one-tile kernels' order: from K = 1024 on, ranges for every count, the first ntiles % 8 XCDs with one tile
+// more.  In plain order each XCD's L2 fetches every panel (FP4 x E3M2 700 x 9842 x 5504, 234 tiles of 128 x 256:
+// 93.9 us in plain order, 62.0 in ranges; bf16 1348 x 9842 x 2432 114 and 101).  Below, the stores count for more,
+// and rows that are not 16-byte aligned are written faster in plain order (FP4 SwiGLU 1348 x 6150 x 128: 24.8 and
+// 26.5 us).  The persistent kernels measure slower with ranges (FP4 pair 4096 x 14336 x 1024: 54 and 60 us).
+__device__ __forceinline__ void tile_of_ranges(unsigned pid, int K, int tiles_m, int tiles_n, int group_m, int& tm,
+                                               int& tn) {
+  const unsigned ntiles = (unsigned)(tiles_m * tiles_n), extra = ntiles % 8u;
+  if (extra == 0 || K >= 1024) {
+    const unsigned xcd = pid % 8u;
+    pid = xcd * (ntiles / 8u) + (xcd < extra ? xcd : extra) + pid / 8u;
+  }
+  tile_at((int)pid, tiles_m, tiles_n, group_m, tm, tn);
 }
 
 __device__ __forceinline__ void store_c(void* c, int cdt, int64_t i, float v) {
