@@ -2,7 +2,8 @@
 // with FP6 (E2M3, E3M2) or FP4 (E2M1) codes on either side, each with E8M0 scales per 32
 // K-elements or unscaled (scale byte 127 = 1.0).  tgm_gemm_mx sends FP4 x FP4 with scales on
 // both sides to its own kernel (tgm_gemm_mx.hip) and every other FP4 / FP6 pair here.  The kernel
-// below takes large products of short K; the others run on the tiles of tgm_gemm_mx_tile.h.
+// below takes products of many tiles: every one of FP4 x FP4, and of short K with an FP6 operand; the others run
+// on the tiles of tgm_gemm_mx_tile.h.
 //
 // Replaces the reference's collective LinAlg GEMM (alexandreteles/tinygrad-dx12
 // src/tinygrad_dx12/renderer/linalg.py:38-124) for two packed operands.  The reference decodes

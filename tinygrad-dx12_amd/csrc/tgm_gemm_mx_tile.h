@@ -22,7 +22,10 @@
 //   E2M3 x E2M3  1001 x 4096: 46.8 -> 29.6   64 x 4096: 41.9 -> 9.9     4096 x 14336: 320 -> 292
 //   FP4 x FP4    1001 x 4096: 27.1 -> 18.1   256 x 14336: 28.4 -> 18.9  17 x 2048 x 1280: 10.2 -> 5.1
 //
-// A stage of the 128 x 128 shape takes 0.7 us, twice its LDS traffic's time; launch, prologue and epilogue are 7 us.
+// A stage (two K steps) of the 128 x 128 shape takes 0.7 us for FP4 x FP4 and 1.0 us for E2M3 x FP4; launch, prologue
+// and epilogue are 7 us.  At 1001 x 4096 x 4096 the latter keeps the LDS active for 29 % of the cycles, almost half of
+// that in bank conflicts of the 24-byte FP6 fragments, and the MFMA pipe busy for 10 % (profiles/one_tile_products.txt):
+// what is left is the chain of barrier, fragment reads and MFMAs of a stage, with one workgroup on a compute unit.
 #pragma once
 
 #include "tgm_gemm_w_tile.h"

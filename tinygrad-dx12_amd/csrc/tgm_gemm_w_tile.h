@@ -23,12 +23,13 @@
 //
 //   FP4   64 x 14336: 42 -> 15      17 x 4096: 39 -> 7.2     512 x 4096: 43 -> 21     512 x 4096 x 14336: 134 -> 66
 //   E2M3  64 x 14336: 51 -> 17      200 x 3000 x 2304: 33 -> 13
-//   INT4 g128  512 x 6144: 74 -> 39     64 x 14336: 71 -> 18     4096 x 4096: 161 -> 135     2048 x 14336: 303 -> 238
+//   INT4 g128  512 x 6144: 74 -> 39     64 x 14336: 68 -> 18     4096 x 4096: 160 -> 139     2048 x 14336: 301 -> 256
 //   INT4 g32   512 x 4096: 96 -> 36     4096 x 4096: 195 -> 173
 //
 // The INT4 products are bound by VALU work beside the MFMAs (12 instructions per 8 codes, and 16 FMAs per
 // MFMA tile and scale group) and by the clock that both together leave: at 4096 x 4096 the MFMA pipe is busy
-// 45 % at 2.07 GHz (the 64 x 64-per-wave kernel before: 34 % at 2.38 GHz, every code decoded twice).
+// 45 % (profiles/one_tile_products.txt) at about 2.06 GHz; the 64 x 64-per-wave kernel before, which decoded every
+// code twice, 34 % at 2.38 GHz.  At 512 x 6144 it is 22 % in one and a half rounds of 64 x 128 tiles.
 //
 // Operand layout in LDS, per K step: the A panel as rows of 256 bytes with 16-byte columns
 // XOR-swizzled by row % 16; the W panel as rows of 64 bytes (FP4, INT4; 16-byte chunks swizzled by
@@ -40,8 +41,8 @@
 // [64 h + 8 j, + 8) of it, so a lane's codes are contiguous.  INT4 takes [16 j + 8 h, + 8): no MFMA spans
 // two groups of 32 or 64, and every group size (and none) sums K in ascending order, so that a rounding
 // does not depend on how a weight's scales are grouped.  (Groups of 128 in the contiguous order, whose
-// codes are two LDS reads instead of four, take the same 38.7 us at 512 x 6144 x 4096 and change the last
-// place of the sums, which the attention of a two-layer decoder prompt grows to 2.4e-3 of its logits.)
+// codes are two LDS reads instead of four, are 3 % faster, 134 against 139 us at 4096 x 4096 x 4096, and change
+// the last place of the sums, which the attention of a two-layer decoder prompt grows to 2.4e-3 of its logits.)
 // INT4 codes become exact f16 values, the MFMAs of a group sum in fp32 and the sum times the group's fp32
 // scale is added to the accumulator.
 #pragma once

@@ -32,8 +32,10 @@
 // rows, V's are transposing reads (ds_read_b64_tr_b16: a 16-lane group reads 4 keys x 16 dims and each
 // lane gets one dim's 4 keys).
 //
-// What bounds it: the MFMAs, 96 per wave and block (three terms each way): at 8 x 512 tokens, 32 heads of
-// 128 they take 28 us.  V was transposed by 2-byte LDS stores from registers before (32 conflicting stores
+// What bounds it: the chain from scores to probabilities to sums within a wave, with two waves per SIMD to
+// overlap.  The MFMAs, 96 per wave and block (three terms each way), would take 28 us of the 87 at 8 x 512
+// tokens, 32 heads of 128; they keep their pipe busy for 25 % of the cycles, and the LDS is active for 5 % of
+// them, without bank conflicts (profiles/prefill_attention.txt).  V was transposed by 2-byte LDS stores from registers before (32 conflicting stores
 // per thread and block), and with them the kernel held 404 registers, one wave per SIMD, so nothing ran
 // beside the softmax: 208 us there and 348 us for one 2048-token prompt, 87 and 146 us now, at the same
 // error (2.2e-7 against 64 bits).
